@@ -221,10 +221,10 @@ struct ObsArgs {
 
 __device__ __forceinline__ bool site_of(const ObsArgs& A, int& x, int& y, int& z, long& s) {
     z = blockIdx.y;
-    long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;  // P sites of a plane: far below 2^32 on any device memory
     if (i >= A.g.P) return false;
-    x = (int)(i % A.g.nx);
-    y = (int)(i / A.g.nx);
+    x = (int)(i % (unsigned)A.g.nx);
+    y = (int)(i / (unsigned)A.g.nx);
     s = i + A.g.P * z;
     return true;
 }
@@ -237,32 +237,60 @@ __device__ __forceinline__ void plaq_full(const double* __restrict__ U, long S, 
 __device__ __forceinline__ double Ev(const double* __restrict__ E, int mu, int a, long s) {
     return E[lidx<long>(kEPlanes, mu * 8 + a, s)];
 }
-__device__ __forceinline__ double Jv(const double* __restrict__ J, int w, int a, long s) {
-    return J[lidx<long>(kJPlanes, w * 8 + a, s)];
+// B_k^2 = 4 Re tr(1 - P_k) of the plaquettes P_0 = P_yz, P_1 = P_zx, P_2 = P_xy rooted at a site, each as Re tr(A B^dag)
+// of its two corner products A = U_m(x) U_n(x+m) and B = U_n(x) U_m(x+n): two matrix products a plaquette, the third is
+// only needed on its diagonal (tr_nd).  What bounds this is how many loads are in flight: the nine links are all read
+// before the first product, at one wavefront per SIMD (286 registers for k_bulk).  Pairs of links at three wavefronts
+// per SIMD took 1.59 ms for the bulk sums at 128 x 128 x 384, three whole plaquettes of four links 0.97, this 0.93
+// (752 B per site, 5.1 TB/s).
+__device__ __forceinline__ void site_b2(const double* __restrict__ U, const Geom& g, int x, int y, int z, long s,
+                                        double* b) {
+    const long sxp = sidx(g, x + 1, y, z), syp = sidx(g, x, y + 1, z), szp = sidx(g, x, y, zup(g, z));
+    M3 X, Y, Z, Yx, Zx, Xy, Zy, Xz, Yz, A, B;
+    ldm<long>(U, kUPlanes, 0, s, X);
+    ldm<long>(U, kUPlanes, 18, s, Y);
+    ldm<long>(U, kUPlanes, 18, sxp, Yx);
+    ldm<long>(U, kUPlanes, 0, syp, Xy);
+    ldm<long>(U, kUPlanes, 36, s, Z);
+    ldm<long>(U, kUPlanes, 36, syp, Zy);
+    ldm<long>(U, kUPlanes, 18, szp, Yz);
+    ldm<long>(U, kUPlanes, 0, szp, Xz);
+    ldm<long>(U, kUPlanes, 36, sxp, Zx);
+    mul_nn(X, Yx, A);
+    mul_nn(Y, Xy, B);
+    b[2] = 4.0 * (3.0 - tr_nd(A, B));
+    mul_nn(Y, Zy, A);
+    mul_nn(Z, Yz, B);
+    b[0] = 4.0 * (3.0 - tr_nd(A, B));
+    mul_nn(Z, Xz, A);
+    mul_nn(X, Zx, B);
+    b[1] = 4.0 * (3.0 - tr_nd(A, B));
 }
-
+// E_mu^2 of a site
+__device__ __forceinline__ double site_e2(const double* __restrict__ E, int mu, long s) {
+    double e[8], v = 0.0;
+    ldv<long>(E, kEPlanes, 8 * mu, s, e);
+#pragma unroll
+    for (int a = 0; a < 8; a++) v += e[a] * e[a];
+    return v;
+}
 // Observables::Bulk (SC/OBSERVABLES/BulkObservables.cpp:65-169): K = 9 (E^2[3], B^2[3], E.J[3])
-__global__ void __launch_bounds__(256) k_bulk(ObsArgs A) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) k_bulk(ObsArgs A) {
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int x, y, z;
     long s;
     if (site_of(A, x, y, z, s)) {
-        const Geom& g = A.g;
-        const long S = g.S;
-        const long sxp = sidx(g, x + 1, y, z), syp = sidx(g, x, y + 1, z), szp = sidx(g, x, y, zup(g, z));
-        M3 Pq;
-        plaq_full(A.U, S, 0, 0, s, 1, sxp, 0, syp, 1, s, Pq);
-        v[5] = 4.0 * retr_one_minus(Pq);  // B2 from Uxy
-        plaq_full(A.U, S, 0, 1, s, 2, syp, 1, szp, 2, s, Pq);
-        v[3] = 4.0 * retr_one_minus(Pq);  // B0 from Uyz
-        plaq_full(A.U, S, 0, 2, s, 0, szp, 2, sxp, 0, s, Pq);
-        v[4] = 4.0 * retr_one_minus(Pq);  // B1 from Uzx
+        site_b2(A.U, A.g, x, y, z, s, v + 3);
+        v[0] = site_e2(A.E, 0, s);
+        v[1] = site_e2(A.E, 1, s);
+        double e[8], jp[8], jm[8];
+        ldv<long>(A.E, kEPlanes, 16, s, e);
+        ldv<long>(A.J, kJPlanes, 8 * JP, s, jp);
+        ldv<long>(A.J, kJPlanes, 8 * JM, s, jm);
+#pragma unroll
         for (int a = 0; a < 8; a++) {
-            const double e0 = Ev(A.E, 0, a, s), e1 = Ev(A.E, 1, a, s), e2 = Ev(A.E, 2, a, s);
-            v[0] += e0 * e0;
-            v[1] += e1 * e1;
-            v[2] += e2 * e2;
-            v[8] += e2 * (Jv(A.J, JP, a, s) - Jv(A.J, JM, a, s)) / kSqrt2;
+            v[2] += e[a] * e[a];
+            v[8] += e[a] * (jp[a] - jm[a]) / kSqrt2;
         }
     }
     block_store<9>(v, A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 9);
@@ -289,9 +317,15 @@ __global__ void __launch_bounds__(256) k_gauss(ObsArgs A) {
         ldm<long>(A.U, kUPlanes, 36, szm, V);
         ldv<long>(A.E, kEPlanes, 16, szm, e);
         inv_adj_mul(V, e, zd);
+        double ex[8], ey[8], ez[8], jp[8], jm[8];
+        ldv<long>(A.E, kEPlanes, 0, s, ex);
+        ldv<long>(A.E, kEPlanes, 8, s, ey);
+        ldv<long>(A.E, kEPlanes, 16, s, ez);
+        ldv<long>(A.J, kJPlanes, 8 * JPS, s, jp);
+        ldv<long>(A.J, kJPlanes, 8 * JMS, s, jm);
+#pragma unroll
         for (int a = 0; a < 8; a++) {
-            const double G = norm * ((Ev(A.E, 0, a, s) - xd[a]) + (Ev(A.E, 1, a, s) - yd[a]) + (Ev(A.E, 2, a, s) - zd[a]) -
-                                     (Jv(A.J, JPS, a, s) + Jv(A.J, JMS, a, s)) / kSqrt2);
+            const double G = norm * ((ex[a] - xd[a]) + (ey[a] - yd[a]) + (ez[a] - zd[a]) - (jp[a] + jm[a]) / kSqrt2);
             v[0] += G * G;
             m[0] = fmax(m[0], fabs(G));
         }
@@ -422,13 +456,13 @@ __global__ void __launch_bounds__(256) k_currents(ObsArgs A) {
     int x, y, z;
     long s;
     if (site_of(A, x, y, z, s)) {
-        for (int a = 0; a < 8; a++) {
-            const double jm = Jv(A.J, JM, a, s), jms = Jv(A.J, JMS, a, s), jp = Jv(A.J, JP, a, s),
-                         jps = Jv(A.J, JPS, a, s);
-            v[0] += jm * jm;
-            v[1] += jms * jms;
-            v[2] += jp * jp;
-            v[3] += jps * jps;
+        const int w[4] = {JM, JMS, JP, JPS};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double j[8];
+            ldv<long>(A.J, kJPlanes, 8 * w[k], s, j);
+#pragma unroll
+            for (int a = 0; a < 8; a++) v[k] += j[a] * j[a];
         }
     }
     block_store<4>(v, A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 4);
@@ -437,15 +471,15 @@ __global__ void __launch_bounds__(256) k_currents(ObsArgs A) {
 // EnergyMomentumTensor::CreateMapBfCollision (SC/OBSERVABLES/EnergyMomentumTensor.cpp:10-77): for each
 // transverse site the energy density summed over z, split at z <= (Nz - 2) / 2 (left) and above (right),
 // from the elementary plaquettes of the current links and the local E.  One thread per (x, y) and chunk of
-// kMapChunk layers; part[(chunk * P + i) * 2 + side].
-constexpr int kMapChunk = 32;
-
-__global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ part) {
+// `chunk` layers; part[(chunk * P + i) * 2 + side].  A layer's loads are a chain of their own, so the chunks are as
+// short as it takes to fill the device (map_chunk): a fixed 32 layers took 183 us at 16 x 16 x 32, one block, and
+// 277 us at 64 x 56 x 96.
+__global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ part, int chunk) {
     const Geom& g = A.g;
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
     if (i >= g.P) return;
-    const int x = (int)(i % g.nx), y = (int)(i / g.nx);
-    const int z0 = blockIdx.y * kMapChunk, z1 = min(z0 + kMapChunk, g.nz);
+    const int x = (int)(i % (unsigned)g.nx), y = (int)(i / (unsigned)g.nx);
+    const int z0 = blockIdx.y * chunk, z1 = min(z0 + chunk, g.nz);
     const int zsplit = (g.nz - 2) / 2;  // (zHigh - 1) / 2 with zHigh = Nz - 1
     const double ac = A.a[0] * A.a[1] * A.a[2];
     double c[3];
@@ -454,22 +488,10 @@ __global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ pa
     double left = 0.0, right = 0.0;
     for (int z = z0; z < z1; z++) {
         const long s = i + g.P * z;
-        const long sxp = sidx(g, x + 1, y, z), syp = sidx(g, x, y + 1, z), szp = sidx(g, x, y, zup(g, z));
-        M3 Pq;
-        plaq_full(A.U, g.S, 0, 0, s, 1, sxp, 0, syp, 1, s, Pq);
-        const double B2 = 4.0 * retr_one_minus(Pq);
-        plaq_full(A.U, g.S, 0, 1, s, 2, syp, 1, szp, 2, s, Pq);
-        const double B0 = 4.0 * retr_one_minus(Pq);
-        plaq_full(A.U, g.S, 0, 2, s, 0, szp, 2, sxp, 0, s, Pq);
-        const double B1 = 4.0 * retr_one_minus(Pq);
-        double E0 = 0.0, E1 = 0.0, E2 = 0.0;
-        for (int a = 0; a < 8; a++) {
-            const double e0 = Ev(A.E, 0, a, s), e1 = Ev(A.E, 1, a, s), e2 = Ev(A.E, 2, a, s);
-            E0 += e0 * e0;
-            E1 += e1 * e1;
-            E2 += e2 * e2;
-        }
-        const double t = 0.5 * (c[0] * E0 + c[1] * E1 + c[2] * E2 + c[0] * B0 + c[1] * B1 + c[2] * B2) * inv_nz;
+        double B[3];
+        site_b2(A.U, g, x, y, z, s, B);
+        const double E0 = site_e2(A.E, 0, s), E1 = site_e2(A.E, 1, s), E2 = site_e2(A.E, 2, s);
+        const double t = 0.5 * (c[0] * E0 + c[1] * E1 + c[2] * E2 + c[0] * B[0] + c[1] * B[1] + c[2] * B[2]) * inv_nz;
         if (z <= zsplit) left += t; else right += t;
     }
     double* o = part + ((long)blockIdx.y * g.P + i) * 2;
@@ -477,29 +499,41 @@ __global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ pa
     o[1] = right;
 }
 
+// layers per thread of k_tmap: up to 32, fewer until the launch has two blocks per CU
+static int map_chunk(const Geom& g) {
+    const long bpp = (g.P + 255) / 256;
+    int chunk = 32;
+    while (chunk > 1 && bpp * ((g.nz + chunk - 1) / chunk) < 512) chunk /= 2;
+    return chunk;
+}
+
 // fixed-order sum of the chunks: out[i * 2 + side] = sum_c part[(c * P + i) * 2 + side]
 __global__ void k_tmap_finalize(const double* __restrict__ part, double* __restrict__ out, long P, int nchunk) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 2 * P) return;
     double acc = 0.0;
+#pragma unroll 8
     for (int c = 0; c < nchunk; c++) acc += part[(long)c * 2 * P + i];
     out[i] = acc;
 }
 
-// per-z fixed-order finalisation: out[z*K + k] = sum_b red[(z*bpp + b)*K + k] (or max for the
-// entries flagged in maxmask)
-__global__ void k_finalize(const double* __restrict__ red, double* __restrict__ out, int nz, int bpp, int K,
-                           unsigned maxmask) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// per-z finalisation: out[z*K + k] = sum_b red[(z*bpp + b)*K + k] (or max for the entries flagged in maxmask).  One
+// wavefront per output: lane l adds the blocks l, l + 64, ... in order, then the lanes are added in a fixed tree, so
+// the result does not depend on scheduling.  One thread per output was a chain of bpp dependent adds on strided
+// loads: 107 us at 256 x 256 x 512 (bpp = 256).
+__global__ void __launch_bounds__(256) k_finalize(const double* __restrict__ red, double* __restrict__ out, int nz,
+                                                  int bpp, int K, unsigned maxmask) {
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= nz * K) return;
-    int z = i / K, k = i % K;
+    const int z = i / K, k = i % K;
     const bool mx = (maxmask >> k) & 1u;
     double acc = 0.0;
-    for (int b = 0; b < bpp; b++) {
-        double v = red[((long)z * bpp + b) * K + k];
+    for (int b = lane; b < bpp; b += 64) {
+        const double v = red[((long)z * bpp + b) * K + k];
         acc = mx ? fmax(acc, v) : acc + v;
     }
-    out[i] = acc;
+    acc = mx ? wave_max(acc) : wave_sum(acc);
+    if (lane == 0) out[i] = acc;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -596,9 +630,10 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     A.bpp = bpp;
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
     hipLaunchKernelGGL(kern, dim3(bpp, g.nz), dim3(256), 0, ctx->stream, A);
+    GL_HIP(ctx, hipGetLastError());
     double* fin = ctx->red + (size_t)g.nz * bpp * K;
     const int n = g.nz * K;
-    hipLaunchKernelGGL(k_finalize, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->red, fin, g.nz, bpp, K, maxmask);
+    hipLaunchKernelGGL(k_finalize, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, ctx->red, fin, g.nz, bpp, K, maxmask);
     per_z.resize(n);
     GL_HIP(ctx, hipMemcpyAsync(per_z.data(), fin, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -843,7 +878,7 @@ int glasma_bulk_noalloc(glasma_ctx* ctx, double* out9) {
     double* fin = ptr + (long)g.nz * bpp * 9;
     double* tot = fin + (long)g.nz * 9;
     hipLaunchKernelGGL(k_bulk, dim3(bpp, g.nz), dim3(256), 0, ctx->stream, A);
-    hipLaunchKernelGGL(k_finalize, dim3((g.nz * 9 + 255) / 256), dim3(256), 0, ctx->stream, ptr, fin, g.nz, bpp, 9, 0u);
+    hipLaunchKernelGGL(k_finalize, dim3((g.nz * 9 + 3) / 4), dim3(256), 0, ctx->stream, ptr, fin, g.nz, bpp, 9, 0u);
     hipLaunchKernelGGL(k_sum_layers, dim3(1), dim3(64), 0, ctx->stream, fin, tot, g.nz, 9);
     GL_HIP(ctx, hipGetLastError());
     GL_HIP(ctx, hipMemcpyAsync(out9, tot, 9 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -952,7 +987,7 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     if (!ctx || !out) return GLASMA_ERR_ARG;
     const Geom& g = ctx->g;
     const int bpp = (int)((g.P + 255) / 256);
-    const int nchunk = (g.nz + kMapChunk - 1) / kMapChunk;
+    const int chunk = map_chunk(g), nchunk = (g.nz + chunk - 1) / chunk;
     int rc = ensure_red(ctx, (size_t)(nchunk + 1) * 2 * g.P);
     if (rc) return rc;
     ObsArgs A;
@@ -965,7 +1000,7 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     A.bpp = bpp;
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
     double* fin = ctx->red + (size_t)nchunk * 2 * g.P;
-    hipLaunchKernelGGL(k_tmap, dim3(bpp, nchunk), dim3(256), 0, ctx->stream, A, ctx->red);
+    hipLaunchKernelGGL(k_tmap, dim3(bpp, nchunk), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
     hipLaunchKernelGGL(k_tmap_finalize, dim3((unsigned)((2 * g.P + 255) / 256)), dim3(256), 0, ctx->stream, ctx->red,
                        fin, (long)g.P, nchunk);
     GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));

@@ -125,6 +125,17 @@ GHD void retr_igen(const M3& V, double* r) {
 // Re tr(1 - V)
 GHD double retr_one_minus(const M3& V) { return 3.0 - V.re[0] - V.re[4] - V.re[8]; }
 
+// Re tr(A B^dag)
+GHD double tr_nd(const M3& A, const M3& B) {
+    double r = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        r = fma(A.re[k], B.re[k], r);
+        r = fma(A.im[k], B.im[k], r);
+    }
+    return r;
+}
+
 // ||V V^dag - 1||_F
 GHD double unitarity_norm(const M3& V) {
     M3 C;
