@@ -208,6 +208,36 @@ __device__ __forceinline__ void block_store_max(double (&v)[K], double* out) {
     }
 }
 
+// Which 256-site chunk of which plane a block of a record kernel takes (block b runs on XCD b % 8, each XCD with its own
+// L2).  band > 0: XCD k takes the bands k, k + 8, ... of `band` consecutive chunks of a plane and walks each through all
+// layers, so that the layers of a band in flight at once share their y and z neighbours in L2; band = 0: XCD k takes the
+// k-th eighth of the chunks, layer by layer.  With chunks dealt to the XCDs in turn the energy-momentum kernel fetched
+// 4.4 times its compulsory bytes at 256 x 256 x 128.
+struct ObsOrder {
+    int bpp, nz, band;
+    unsigned n, per;  // blocks, blocks per XCD (far below 2^32 on any device memory)
+};
+static ObsOrder obs_order(int bpp, int nz) {
+    const unsigned n = (unsigned)bpp * (unsigned)nz;
+    ObsOrder o = {bpp, nz, 0, n, (n + kXcds - 1) / kXcds};
+    for (int b = 1; b <= 16; b++)
+        if (bpp % b == 0 && bpp / b % kXcds == 0) o.band = b;
+    return o;
+}
+__device__ __forceinline__ bool obs_block(const ObsOrder& o, int& chunk, int& z) {
+    const unsigned k = blockIdx.x % kXcds, i = blockIdx.x / kXcds;
+    if (o.band) {
+        const unsigned per = (unsigned)o.band * o.nz, m = i / per, r = i - m * per;
+        z = (int)(r / o.band);
+        chunk = (int)((m * kXcds + k) * o.band + r % o.band);
+        return true;
+    }
+    const unsigned b = k * o.per + i;
+    z = (int)(b / o.bpp);
+    chunk = (int)(b % o.bpp);
+    return b < o.n;
+}
+
 struct ObsArgs {
     const double* __restrict__ U;
     const double* __restrict__ UOld;
@@ -216,12 +246,17 @@ struct ObsArgs {
     double* __restrict__ red;
     Geom g;
     int bpp;  // blocks per plane
+    ObsOrder ord;
     double a[3];
 };
 
-__device__ __forceinline__ bool site_of(const ObsArgs& A, int& x, int& y, int& z, long& s) {
-    z = blockIdx.y;
-    const unsigned i = blockIdx.x * 256 + threadIdx.x;  // P sites of a plane: far below 2^32 on any device memory
+// the block's place for its partial sums (null: no chunk) and the thread's site (false: none)
+template <int K>
+__device__ __forceinline__ double* part_of(const ObsArgs& A, int& chunk, int& z) {
+    return obs_block(A.ord, chunk, z) ? A.red + ((long)z * A.bpp + chunk) * K : nullptr;
+}
+__device__ __forceinline__ bool site_of(const ObsArgs& A, int chunk, int& x, int& y, int z, long& s) {
+    const unsigned i = chunk * 256u + threadIdx.x;  // P sites of a plane: far below 2^32 on any device memory
     if (i >= A.g.P) return false;
     x = (int)(i % (unsigned)A.g.nx);
     y = (int)(i / (unsigned)A.g.nx);
@@ -277,9 +312,11 @@ __device__ __forceinline__ double site_e2(const double* __restrict__ E, int mu, 
 // Observables::Bulk (SC/OBSERVABLES/BulkObservables.cpp:65-169): K = 9 (E^2[3], B^2[3], E.J[3])
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) k_bulk(ObsArgs A) {
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int x, y, z;
+    int chunk, x, y, z;
     long s;
-    if (site_of(A, x, y, z, s)) {
+    double* const out = part_of<9>(A, chunk, z);
+    if (!out) return;
+    if (site_of(A, chunk, x, y, z, s)) {
         site_b2(A.U, A.g, x, y, z, s, v + 3);
         v[0] = site_e2(A.E, 0, s);
         v[1] = site_e2(A.E, 1, s);
@@ -293,16 +330,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
             v[8] += e[a] * (jp[a] - jm[a]) / kSqrt2;
         }
     }
-    block_store<9>(v, A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 9);
+    block_store<9>(v, out);
 }
 
 // COMPUTE_GAUSS_VIOLATION (SC/CALC/GaussViolation.cpp:13-23): K = 2 sums (sum G^2) + 1 max (|G^a|)
 __global__ void __launch_bounds__(256) k_gauss(ObsArgs A) {
     double v[1] = {0.0};
     double m[1] = {0.0};
-    int x, y, z;
+    int chunk, x, y, z;
     long s;
-    if (site_of(A, x, y, z, s)) {
+    double* const out = part_of<2>(A, chunk, z);
+    if (!out) return;
+    if (site_of(A, chunk, x, y, z, s)) {
         const Geom& g = A.g;
         const long sxm = sidx(g, x - 1, y, z), sym = sidx(g, x, y - 1, z), szm = sidx(g, x, y, zdn(g, z));
         const double norm = 1.0 / (A.a[0] * A.a[1] * A.a[2]);
@@ -330,7 +369,6 @@ __global__ void __launch_bounds__(256) k_gauss(ObsArgs A) {
             m[0] = fmax(m[0], fabs(G));
         }
     }
-    double* out = A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 2;
     block_store<1>(v, out);
     block_store_max<1>(m, out + 1);
 }
@@ -338,9 +376,11 @@ __global__ void __launch_bounds__(256) k_gauss(ObsArgs A) {
 // Unitarity (SC/OBSERVABLES/UnitarityViolation.cpp:13-51): sum of squares and max
 __global__ void __launch_bounds__(256) k_unitarity(ObsArgs A) {
     double v[1] = {0.0}, m[1] = {0.0};
-    int x, y, z;
+    int chunk, x, y, z;
     long s;
-    if (site_of(A, x, y, z, s)) {
+    double* const out = part_of<2>(A, chunk, z);
+    if (!out) return;
+    if (site_of(A, chunk, x, y, z, s)) {
         for (int mu = 0; mu < 3; mu++) {
             M3 V;
             ldm<long>(A.U, kUPlanes, 18 * mu, s, V);
@@ -349,7 +389,6 @@ __global__ void __launch_bounds__(256) k_unitarity(ObsArgs A) {
             m[0] = fmax(m[0], n);
         }
     }
-    double* out = A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 2;
     block_store<1>(v, out);
     block_store_max<1>(m, out + 1);
 }
@@ -359,9 +398,11 @@ __global__ void __launch_bounds__(256) k_unitarity(ObsArgs A) {
 // x and x - mu (colour vectors parallel transported with the current U).  K = 10.
 __global__ void __launch_bounds__(256) k_emt(ObsArgs A) {
     double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int x, y, z;
+    int chunk, x, y, z;
     long s;
-    if (site_of(A, x, y, z, s)) {
+    double* const out = part_of<10>(A, chunk, z);
+    if (!out) return;
+    if (site_of(A, chunk, x, y, z, s)) {
         const Geom& g = A.g;
         const long S = g.S;
         const int zp = zup(g, z), zm = zdn(g, z);
@@ -446,16 +487,18 @@ __global__ void __launch_bounds__(256) k_emt(ObsArgs A) {
         v[8] = (q1 * q2 * dot(E1, E2) + q1 * q2 * dot(B1, B2)) * inv;
         v[9] = (q2 * q0 * dot(E2, E0) + q2 * q0 * dot(B2, B0)) * inv;
     }
-    block_store<10>(v, A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 10);
+    block_store<10>(v, out);
 }
 
 // IO::SaveTransverselyIntegratedCurrents (SC/IO/SaveConfiguration.cpp:160-204): per layer
 // sum_{x,y,a} of Jm^2, JmStat^2, Jp^2, JpStat^2.  K = 4.
 __global__ void __launch_bounds__(256) k_currents(ObsArgs A) {
     double v[4] = {0, 0, 0, 0};
-    int x, y, z;
+    int chunk, x, y, z;
     long s;
-    if (site_of(A, x, y, z, s)) {
+    double* const out = part_of<4>(A, chunk, z);
+    if (!out) return;
+    if (site_of(A, chunk, x, y, z, s)) {
         const int w[4] = {JM, JMS, JP, JPS};
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -465,7 +508,7 @@ __global__ void __launch_bounds__(256) k_currents(ObsArgs A) {
             for (int a = 0; a < 8; a++) v[k] += j[a] * j[a];
         }
     }
-    block_store<4>(v, A.red + ((long)blockIdx.y * A.bpp + blockIdx.x) * 4);
+    block_store<4>(v, out);
 }
 
 // EnergyMomentumTensor::CreateMapBfCollision (SC/OBSERVABLES/EnergyMomentumTensor.cpp:10-77): for each
@@ -476,10 +519,12 @@ __global__ void __launch_bounds__(256) k_currents(ObsArgs A) {
 // 277 us at 64 x 56 x 96.
 __global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ part, int chunk) {
     const Geom& g = A.g;
-    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    int pc, zc;
+    if (!obs_block(A.ord, pc, zc)) return;
+    const unsigned i = pc * 256u + threadIdx.x;
     if (i >= g.P) return;
     const int x = (int)(i % (unsigned)g.nx), y = (int)(i / (unsigned)g.nx);
-    const int z0 = blockIdx.y * chunk, z1 = min(z0 + chunk, g.nz);
+    const int z0 = zc * chunk, z1 = min(z0 + chunk, g.nz);
     const int zsplit = (g.nz - 2) / 2;  // (zHigh - 1) / 2 with zHigh = Nz - 1
     const double ac = A.a[0] * A.a[1] * A.a[2];
     double c[3];
@@ -494,7 +539,7 @@ __global__ void __launch_bounds__(256) k_tmap(ObsArgs A, double* __restrict__ pa
         const double t = 0.5 * (c[0] * E0 + c[1] * E1 + c[2] * E2 + c[0] * B[0] + c[1] * B[1] + c[2] * B[2]) * inv_nz;
         if (z <= zsplit) left += t; else right += t;
     }
-    double* o = part + ((long)blockIdx.y * g.P + i) * 2;
+    double* o = part + ((long)zc * g.P + i) * 2;
     o[0] = left;
     o[1] = right;
 }
@@ -628,8 +673,9 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     A.red = ctx->red;
     A.g = g;
     A.bpp = bpp;
+    A.ord = obs_order(bpp, g.nz);
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
-    hipLaunchKernelGGL(kern, dim3(bpp, g.nz), dim3(256), 0, ctx->stream, A);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A);
     GL_HIP(ctx, hipGetLastError());
     double* fin = ctx->red + (size_t)g.nz * bpp * K;
     const int n = g.nz * K;
@@ -874,10 +920,11 @@ int glasma_bulk_noalloc(glasma_ctx* ctx, double* out9) {
     A.red = ptr;
     A.g = g;
     A.bpp = bpp;
+    A.ord = obs_order(bpp, g.nz);
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
     double* fin = ptr + (long)g.nz * bpp * 9;
     double* tot = fin + (long)g.nz * 9;
-    hipLaunchKernelGGL(k_bulk, dim3(bpp, g.nz), dim3(256), 0, ctx->stream, A);
+    hipLaunchKernelGGL(k_bulk, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A);
     hipLaunchKernelGGL(k_finalize, dim3((g.nz * 9 + 3) / 4), dim3(256), 0, ctx->stream, ptr, fin, g.nz, bpp, 9, 0u);
     hipLaunchKernelGGL(k_sum_layers, dim3(1), dim3(64), 0, ctx->stream, fin, tot, g.nz, 9);
     GL_HIP(ctx, hipGetLastError());
@@ -998,9 +1045,10 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     A.red = nullptr;
     A.g = g;
     A.bpp = bpp;
+    A.ord = obs_order(bpp, nchunk);
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
     double* fin = ctx->red + (size_t)nchunk * 2 * g.P;
-    hipLaunchKernelGGL(k_tmap, dim3(bpp, nchunk), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
+    hipLaunchKernelGGL(k_tmap, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
     hipLaunchKernelGGL(k_tmap_finalize, dim3((unsigned)((2 * g.P + 255) / 256)), dim3(256), 0, ctx->stream, ctx->red,
                        fin, (long)g.P, nchunk);
     GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
