@@ -39,6 +39,21 @@ void hc_tile_sites(const int* n, int mode, int bpb, int bw, int bh, int nbx, int
     for (long b = 0; b < nblocks; b++) out[b] = tile_site(g, m, b);
 }
 
+// the x neighbours that the row copy of the tile starting at site `first` holds (site.h row_slots, halo_site): for every
+// lane the sites in the slots of x + 1 and x - 1
+void hc_row_neighbours(const int* n, long first, long* xp, long* xm) {
+    Geom g = {n[0], n[1], n[2], 0, (long)n[0] * n[1] * n[2], (long)n[0] * n[1]};
+    long slot[kTile + 4];
+    for (int l = 0; l < kTile; l++) slot[l + 1] = first + l;
+    const int x0 = (int)(first % g.nx), where[4] = {0, kTile + 1, kTile + 2, kTile + 3};
+    for (int h = 0; h < 4; h++) slot[where[h]] = halo_site(g, first, x0, h);
+    for (int l = 0; l < kTile; l++) {
+        const RowSlots r = row_slots(g, l, (int)((first + l) % g.nx));
+        xp[l] = slot[r.sp];
+        xm[l] = slot[r.sm];
+    }
+}
+
 // One fused leapfrog step over tiled device-layout arrays, sequentially over sites.
 void hc_step(const int* n, const double* a, int bc, double dt, const double* U, double* Un, double* E,
              const double* J, double* Jn, double* UOld) {

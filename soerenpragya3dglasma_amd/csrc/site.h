@@ -236,29 +236,42 @@ GHD void plaq_mat(const double* __restrict__ U, int kind, int m1, I s1, int m2, 
 // Order in which the blocks of a step visit the tiles.  Workgroups are dealt to the 8 XCDs round-robin
 // (block b runs on XCD b % 8), each XCD with its own L2.
 //   mode 0: linear, tile b.
-//   mode 1: XCD k owns the k-th band of P/8 sites of every z plane and walks the planes in order.
+//   mode 1: XCD k owns the k-th band (bpb tiles) of every z plane and walks the planes in order.  A plane counts as
+//           8 bpb tiles, the multiple of 8 nearest to its own P/64: where that is not exact the bands shift by a tile or
+//           so from one plane to the next, and the tiles left at the end are taken in linear order.
 //   mode 2: column bands of bw tiles (64 x-sites each) by bh rows; XCD k takes bands k, k+8, ... and
 //           walks each band through all z planes before the next one, so the few planes of one band that
 //           are in flight at once share their z neighbours in L2.
-//   mode 3: z slabs: XCD k takes the k-th eighth of the tiles in linear order (bpb tiles: whole planes and their
-//           y neighbours on one XCD, for planes whose tile count is not a multiple of 8).
+//   mode 3: z slabs: XCD k takes the k-th eighth of the tiles in linear order (bpb tiles, the first nbx XCDs one more:
+//           whole planes and their y neighbours on one XCD, for planes whose tile count is not a multiple of 8).
 constexpr int kXcds = 8;
 
-// whether the step can take its row operands from an LDS copy of the tile: nx a multiple of 64 (a tile is part
-// of one row), a divisor of 64 (whole rows), or a tile spans at most two row segments (every tile start x0 =
-// 64 t mod nx, a multiple of gcd(64, nx), has x0 + 64 <= 2 nx, i.e. nx >= 64 - gcd(64, nx); nx = 48 and 96
-// among others) with no partial last tile
-GHD int gcd64(int n) {
-    int g = kTile;
-    while (n % g) g >>= 1;
-    return g;
+// how the step's tiles lie on the lattice rows: 1: whole rows per tile (nx divides 64) or one row segment (nx a multiple
+// of 64); 2: any other nx, where a tile starts and ends anywhere in a row
+GHD int row_form(const Geom& g) { return g.nx % kTile == 0 || kTile % g.nx == 0 ? 1 : 2; }
+// LDS slots of the x + 1 and x - 1 neighbours of a tile's lane (row_form 2): slot 1 + lane for a site of the tile, and
+// four halo slots: 0 left of lane 0, 65 right of lane 63, 66 right of the end of the tile's first row when that row starts
+// before the tile (x = nx - 1 -> 0), 67 left of the start of its last row when that row ends after the tile
+struct RowSlots {
+    int sp, sm;
+};
+GHD RowSlots row_slots(const Geom& g, int lane, int x) {
+    const int r = x + 1 == g.nx ? lane + 1 - g.nx : lane + 1, l = x == 0 ? lane + g.nx - 1 : lane - 1;
+    RowSlots s;
+    s.sp = r < 0 ? kTile + 2 : r + 1;  // r = 64: slot 65
+    s.sm = l >= kTile ? kTile + 3 : l + 1;
+    return s;
 }
-// 0: the plain form; 1: the row-staged form with whole rows or one row segment per tile; 2: two segments
-GHD int row_form(const Geom& g) {
-    if (g.nx % kTile == 0 || kTile % g.nx == 0) return 1;
-    return g.nx >= kTile - gcd64(g.nx) && g.S % kTile == 0 ? 2 : 0;
+// the site held by halo slot h (0: slot 0, 1: slot 65, 2: slot 66, 3: slot 67) of the tile starting at `first`, whose
+// first site has x = x0; a site of the lattice also where the tile does not need the slot
+GHD long halo_site(const Geom& g, long first, int x0, int h) {
+    if (h == 0) return first > 0 ? first - 1 : 0;
+    if (h == 2) return first - x0;
+    const long end = first + kTile - 1;  // lane 63
+    const long s = h == 1 ? end + 1 : end - (x0 + kTile - 1) % g.nx + g.nx - 1;
+    return s < g.S ? s : g.S - 1;
 }
-GHD bool row_tiles(const Geom& g) { return row_form(g) != 0; }
+
 struct TileMap {
     int mode, bpb;
     int bw, bh, nbx, tpbp;
@@ -268,10 +281,11 @@ struct TileMap {
 GHD long tile_site(const Geom& g, const TileMap& m, long b) {
     if (m.mode == 0) return b * kTile;
     const long k = b % kXcds, i = b / kXcds;
-    if (m.mode == 3) return (k * m.bpb + i) * kTile;
+    if (m.mode == 3) return (k * m.bpb + (k < m.nbx ? k : m.nbx) + i) * kTile;
     if (m.mode == 1) {
-        const long z = i / m.bpb, j = i % m.bpb;
-        return z * g.P + k * (g.P / kXcds) + j * kTile;
+        const long z = i / m.bpb, j = i % m.bpb, n = (long)kXcds * m.bpb;  // n: tiles counted as a plane
+        if ((z + 1) * n * kTile > pad_sites(g.S)) return b * kTile;
+        return (z * n + k * m.bpb + j) * kTile;
     }
     const long per_band = (long)g.nz * m.tpbp;
     const long mb = i / per_band, r = i - mb * per_band;
