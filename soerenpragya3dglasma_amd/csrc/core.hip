@@ -264,14 +264,6 @@ __device__ __forceinline__ bool site_of(const ObsArgs& A, int chunk, int& x, int
     return true;
 }
 
-__device__ __forceinline__ void plaq_full(const double* __restrict__ U, long S, int kind, int m1, long s1, int m2,
-                                          long s2, int m3, long s3, int m4, long s4, M3& Pq) {
-    (void)S;
-    plaq_mat<long>(U, kind, m1, s1, m2, s2, m3, s3, m4, s4, Pq);
-}
-__device__ __forceinline__ double Ev(const double* __restrict__ E, int mu, int a, long s) {
-    return E[lidx<long>(kEPlanes, mu * 8 + a, s)];
-}
 // B_k^2 = 4 Re tr(1 - P_k) of the plaquettes P_0 = P_yz, P_1 = P_zx, P_2 = P_xy rooted at a site, each as Re tr(A B^dag)
 // of its two corner products A = U_m(x) U_n(x+m) and B = U_n(x) U_m(x+n): two matrix products a plaquette, the third is
 // only needed on its diagonal (tr_nd).  What bounds this is how many loads are in flight: the nine links are all read
@@ -393,9 +385,88 @@ __global__ void __launch_bounds__(256) k_unitarity(ObsArgs A) {
     block_store_max<1>(m, out + 1);
 }
 
+// The same plane of links at several sites, element by element: sites that differ by one in x share their cache lines,
+// which then come once from L2.
+template <int N>
+__device__ __forceinline__ void ld_group(const double* __restrict__ U, int mu, const long (&s)[N], M3 (&M)[N]) {
+    const double* q[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) q[i] = site_ptr<long>(U, kUPlanes, 18 * mu, s[i]);
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const d2_t v = ld2(q[i] + k * 2 * kTile);
+            M[i].re[k] = v.x;
+            M[i].im[k] = v.y;
+        }
+}
+
+// Re tr(A B)
+__device__ __forceinline__ double tr_nn(const M3& A, const M3& B) {
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            r = fma(A.re[mi(i, j)], B.re[mi(j, i)], r);
+            r = fma(-A.im[mi(i, j)], B.im[mi(j, i)], r);
+        }
+    return r;
+}
+
+// The clover of the plane (m, n) at s: b = 2 Re tr(i t^a C) and b2 = 4 Re tr(1 - C) of the mean C of its four leaves
+// (SC/SUNc/AdvancedOperations.cpp:35-40).  With the spokes a = U_m(x), b = U_n(x), c = U_m(x-m), d = U_n(x-n) and the
+// outer corners A1 = U_n(x+m) U_m^dag(x+n), A2 = U_m^dag(x-m+n) U_n^dag(x-m), A3 = U_m(x-n) U_n(x-n+m),
+// A4 = U_n^dag(x-m-n) U_m(x-m-n) the leaves are a A1 b^dag, b A2 c, d^dag A3 a^dag and c^dag A4 d.  Re tr(i t^a X^dag) =
+// -Re tr(i t^a X), so the projection is that of a (A1 b^dag - A3^dag d) + (b A2 - d^dag A4^dag) c, and the traces add with
+// the other signs: ten products and twelve links (four leaves on their own: twelve and sixteen).
+__device__ __forceinline__ void clover(const double* __restrict__ W, const Geom& g, int m, int n, int x, int y, int z,
+                                       double* b, double& b2) {
+    auto at = [&](int sm, int sn) { return nbr<long>(g, x, y, z, m, sm, n, sn); };
+    M3 Y1, Z1, Y, T;
+    {
+        M3 G[3], H[2], A;
+        ld_group<3>(W, n, {at(0, 0), at(1, 0), at(-1, 0)}, G);
+        ld_group<2>(W, m, {at(0, 1), at(-1, 1)}, H);
+        mul_nd(G[1], H[0], A);
+        mul_nd(A, G[0], Y1);
+        mul_dd(H[1], G[2], A);
+        mul_nn(G[0], A, Z1);
+    }
+    M3 Y2, Z2;
+    {
+        M3 G[3], H[2], A;
+        ld_group<3>(W, n, {at(0, -1), at(1, -1), at(-1, -1)}, G);
+        ld_group<2>(W, m, {at(0, -1), at(-1, -1)}, H);
+        mul_nn(H[0], G[1], A);
+        mul_dn(A, G[0], Y2);
+        mul_dn(G[2], H[1], A);
+        mul_dd(G[0], A, Z2);
+    }
+    M3 S[2];
+    ld_group<2>(W, m, {at(0, 0), at(-1, 0)}, S);
+    double t = tr_nn(S[0], Y1) + tr_nn(S[0], Y2) + tr_nn(Z1, S[1]) + tr_nn(Z2, S[1]);
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        Y.re[k] = Y1.re[k] - Y2.re[k];
+        Y.im[k] = Y1.im[k] - Y2.im[k];
+        Z1.re[k] -= Z2.re[k];
+        Z1.im[k] -= Z2.im[k];
+    }
+    double f[8];
+    retr_igen_prod(S[0], Y, b);
+    retr_igen_prod(Z1, S[1], f);
+#pragma unroll
+    for (int a = 0; a < 8; a++) b[a] = 0.5 * (b[a] + f[a]);
+    b2 = 4.0 * (3.0 - 0.25 * t);
+}
+
 // EnergyMomentumTensor::CreateMap (SC/OBSERVABLES/EnergyMomentumTensor.cpp:92-170) with
 // COMPUTE_AVG_FIELD_STRENGTH (SC/CALC/AvgFieldStrength.cpp:68-145): clover B on UOld, E averaged over
 // x and x - mu (colour vectors parallel transported with the current U).  K = 10.
+// What bounds it is the links' way from L2: sixteen links a clover in four separate leaves took 16.5 ms at
+// 256 x 256 x 512.
 __global__ void __launch_bounds__(256) k_emt(ObsArgs A) {
     double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     int chunk, x, y, z;
@@ -404,69 +475,32 @@ __global__ void __launch_bounds__(256) k_emt(ObsArgs A) {
     if (!out) return;
     if (site_of(A, chunk, x, y, z, s)) {
         const Geom& g = A.g;
-        const long S = g.S;
-        const int zp = zup(g, z), zm = zdn(g, z);
         const long s0 = s;
-        const long sxp = sidx(g, x + 1, y, z), sxm = sidx(g, x - 1, y, z), syp = sidx(g, x, y + 1, z),
-                   sym = sidx(g, x, y - 1, z), szp = sidx(g, x, y, zp), szm = sidx(g, x, y, zm);
-        const long s_mxpy = sidx(g, x - 1, y + 1, z), s_xpmy = sidx(g, x + 1, y - 1, z);
-        const long s_ympz = sidx(g, x, y - 1, zp), s_ypmz = sidx(g, x, y + 1, zm);
-        const long s_xpmz = sidx(g, x + 1, y, zm), s_mxpz = sidx(g, x - 1, y, zp);
-        const long s_mxmy = sidx(g, x - 1, y - 1, z), s_mymz = sidx(g, x, y - 1, zm), s_mxmz = sidx(g, x - 1, y, zm);
-        const double* W = A.UOld;
-        M3 Pq, Axy, Ayz, Azx;
-        // clover averages, SC/SUNc/AdvancedOperations.cpp:35-40 (0.25 * (P1 + P2 + P3 + P4))
-        auto acc4 = [&](M3& Av, const M3& p1, const M3& p2, const M3& p3, const M3& p4) {
-            for (int k = 0; k < 9; k++) {
-                Av.re[k] = 0.25 * (p1.re[k] + p2.re[k] + p3.re[k] + p4.re[k]);
-                Av.im[k] = 0.25 * (p1.im[k] + p2.im[k] + p3.im[k] + p4.im[k]);
+        const long sxm = sidx(g, x - 1, y, z), sym = sidx(g, x, y - 1, z), szm = sidx(g, x, y, zdn(g, z));
+        double B0[8], B1[8], B2[8], B0S, B1S, B2S;
+        clover(A.UOld, g, 0, 1, x, y, z, B2, B2S);
+        clover(A.UOld, g, 0, 2, x, y, z, B1, B1S);  // the xz plane: its leaves are the zx plane's, reversed
+#pragma unroll
+        for (int a = 0; a < 8; a++) B1[a] = -B1[a];
+        clover(A.UOld, g, 1, 2, x, y, z, B0, B0S);
+        double E0[8], E1[8], E2[8], E0S, E1S, E2S;
+        auto avg = [&](int mu, long sm, double* Em, double& es) {
+            M3 V;
+            double e[8], ed[8];
+            ldm<long>(A.U, kUPlanes, 18 * mu, sm, V);
+            ldv<long>(A.E, kEPlanes, 8 * mu, sm, e);
+            ldv<long>(A.E, kEPlanes, 8 * mu, s0, Em);
+            inv_adj_mul(V, e, ed);
+            es = 0.0;
+#pragma unroll
+            for (int a = 0; a < 8; a++) {
+                es += 0.5 * (Em[a] * Em[a] + e[a] * e[a]);
+                Em[a] = 0.5 * (Em[a] + ed[a]);
             }
         };
-        {
-            M3 a1, a2, a3, a4;
-            plaq_full(W, S, 0, 0, s0, 1, sxp, 0, syp, 1, s0, a1);        // Uxy
-            plaq_full(W, S, 1, 1, s0, 0, s_mxpy, 1, sxm, 0, sxm, a2);    // UMxy
-            plaq_full(W, S, 2, 1, sym, 0, sym, 1, s_xpmy, 0, s0, a3);    // UxMy
-            plaq_full(W, S, 3, 0, sxm, 1, s_mxmy, 0, s_mxmy, 1, sym, a4);  // UMxMy
-            acc4(Axy, a1, a2, a3, a4);
-            plaq_full(W, S, 0, 1, s0, 2, syp, 1, szp, 2, s0, a1);        // Uyz
-            plaq_full(W, S, 1, 2, s0, 1, s_ympz, 2, sym, 1, sym, a2);    // UMyz
-            plaq_full(W, S, 2, 2, szm, 1, szm, 2, s_ypmz, 1, s0, a3);    // UyMz
-            plaq_full(W, S, 3, 1, sym, 2, s_mymz, 1, s_mymz, 2, szm, a4);  // UMyMz
-            acc4(Ayz, a1, a2, a3, a4);
-            plaq_full(W, S, 0, 2, s0, 0, szp, 2, sxp, 0, s0, a1);        // Uzx
-            plaq_full(W, S, 1, 0, s0, 2, s_xpmz, 0, szm, 2, szm, a2);    // UMzx
-            plaq_full(W, S, 2, 0, sxm, 2, sxm, 0, s_mxpz, 2, s0, a3);    // UzMx
-            plaq_full(W, S, 3, 2, szm, 0, s_mxmz, 2, s_mxmz, 0, sxm, a4);  // UMzMx
-            acc4(Azx, a1, a2, a3, a4);
-        }
-        (void)Pq;
-        double B0[8], B1[8], B2[8];
-        retr_igen(Ayz, B0);
-        retr_igen(Azx, B1);
-        retr_igen(Axy, B2);
-        for (int a = 0; a < 8; a++) { B0[a] *= 2.0; B1[a] *= 2.0; B2[a] *= 2.0; }
-        const double B0S = 4.0 * retr_one_minus(Ayz), B1S = 4.0 * retr_one_minus(Azx), B2S = 4.0 * retr_one_minus(Axy);
-        double E0[8], E1[8], E2[8], ed[8], e[8];
-        double E0S = 0, E1S = 0, E2S = 0;
-        M3 V;
-        const long sm[3] = {sxm, sym, szm};
-        for (int mu = 0; mu < 3; mu++) {
-            double* Em = mu == 0 ? E0 : (mu == 1 ? E1 : E2);
-            ldm<long>(A.U, kUPlanes, 18 * mu, sm[mu], V);
-            ldv<long>(A.E, kEPlanes, 8 * mu, sm[mu], e);
-            inv_adj_mul(V, e, ed);
-            double es = 0.0;
-            for (int a = 0; a < 8; a++) {
-                const double eh = Ev(A.E, mu, a, s0);
-                Em[a] = 0.5 * (eh + ed[a]);
-            }
-            for (int a = 0; a < 8; a++) {
-                const double eh = Ev(A.E, mu, a, s0);
-                es += 0.5 * (eh * eh + e[a] * e[a]);
-            }
-            if (mu == 0) E0S = es; else if (mu == 1) E1S = es; else E2S = es;
-        }
+        avg(0, sxm, E0, E0S);
+        avg(1, sym, E1, E1S);
+        avg(2, szm, E2, E2S);
         double q0 = A.a[0] / (A.a[0] * A.a[1] * A.a[2]), q1 = A.a[1] / (A.a[0] * A.a[1] * A.a[2]),
                q2 = A.a[2] / (A.a[0] * A.a[1] * A.a[2]);
         const double inv = 1.0 / (double)g.P;
