@@ -44,73 +44,6 @@ int ensure_fftbuf(glasma_ctx* ctx, size_t doubles) {
     return 0;
 }
 
-// ------------------------------------------------------------------------------------------------
-// AoS <-> SoA transposition (record of R doubles per site)
-// ------------------------------------------------------------------------------------------------
-// record of R doubles per site (AoS) <-> planes p0 .. p0+R-1 of a tiled field with NP planes
-__global__ void k_aos_to_soa(const double* __restrict__ aos, double* __restrict__ soa, long S, int R, int NP, int p0) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S * R) return;
-    long s = i / R;
-    int j = (int)(i % R);
-    soa[lidx<long>(NP, p0 + j, s)] = aos[i];
-}
-__global__ void k_soa_to_aos(const double* __restrict__ soa, double* __restrict__ aos, long S, int R, int NP, int p0) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S * R) return;
-    long s = i / R;
-    int j = (int)(i % R);
-    aos[i] = soa[lidx<long>(NP, p0 + j, s)];
-}
-
-int upload_aos(glasma_ctx* ctx, const double* host_with_ghosts, double* dev_soa, int R, int NP, int p0) {
-    if (NP < 0) NP = R;
-    const long S = ctx->g.S, P = ctx->g.P;
-    double* tmp = nullptr;
-    GL_HIP(ctx, hipMalloc(&tmp, (size_t)S * R * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(tmp, host_with_ghosts + (size_t)P * R, (size_t)S * R * sizeof(double),
-                                  hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) {
-        long n = S * R;
-        hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, tmp, dev_soa, S, R,
-                           NP, p0);
-        e = hipStreamSynchronize(ctx->stream);
-    }
-    (void)hipFree(tmp);
-    if (e != hipSuccess) return hip_fail(ctx, e, "upload_aos");
-    return 0;
-}
-
-// fill the two ghost layers of a host AoS array as SynchronizeGhostCells does
-void host_sync_ghosts(const glasma_ctx* ctx, double* h, int R) {
-    const long P = ctx->g.P * R;
-    const int nz = ctx->g.nz;
-    if (ctx->p.bc_z == 0) {
-        std::memcpy(h, h + P, P * sizeof(double));
-        std::memcpy(h + (long)(nz + 1) * P, h + (long)nz * P, P * sizeof(double));
-    } else {
-        std::memcpy(h, h + (long)nz * P, P * sizeof(double));
-        std::memcpy(h + (long)(nz + 1) * P, h + P, P * sizeof(double));
-    }
-}
-
-int download_aos(glasma_ctx* ctx, const double* dev_soa, double* host_with_ghosts, int R, int NP, int p0) {
-    if (NP < 0) NP = R;
-    const long S = ctx->g.S, P = ctx->g.P;
-    double* tmp = nullptr;
-    GL_HIP(ctx, hipMalloc(&tmp, (size_t)S * R * sizeof(double)));
-    long n = S * R;
-    hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, dev_soa, tmp, S, R, NP,
-                       p0);
-    hipError_t e = hipMemcpyAsync(host_with_ghosts + (size_t)P * R, tmp, (size_t)S * R * sizeof(double),
-                                  hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess) return hip_fail(ctx, e, "download_aos");
-    host_sync_ghosts(ctx, host_with_ghosts, R);
-    return 0;
-}
-
 static int upload_j(glasma_ctx* ctx, const double* h, double* J, int w) { return upload_aos(ctx, h, J, 8, kJPlanes, 8 * w); }
 static int download_j(glasma_ctx* ctx, const double* J, double* h, int w) {
     return download_aos(ctx, J, h, 8, kJPlanes, 8 * w);
@@ -753,6 +686,7 @@ int glasma_create(const glasma_params* p, glasma_ctx** out) {
             return create_fail(GLASMA_ERR_ARG, "glasma_create: lattice sizes and spacings must be positive");
     if (p->bc_z != 0 && p->bc_z != 1) return create_fail(GLASMA_ERR_ARG, "glasma_create: bc_z must be 0 or 1");
     glasma_ctx* ctx = new glasma_ctx();
+    stage_context_created();
     ctx->p = *p;
     ctx->g.nx = p->n[0];
     ctx->g.ny = p->n[1];
@@ -804,6 +738,7 @@ int glasma_destroy(glasma_ctx* ctx) {
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     if (ctx->stream2) hipStreamDestroy(ctx->stream2);
     delete ctx;
+    stage_context_destroyed();
     return 0;
 }
 

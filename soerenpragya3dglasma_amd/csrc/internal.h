@@ -88,6 +88,9 @@ int reset_fields(glasma_ctx* ctx);
 // tiled device field with NP planes (NP < 0: NP = R)
 int upload_aos(glasma_ctx* ctx, const double* host_with_ghosts, double* dev_soa, int R, int NP = -1, int p0 = 0);
 int download_aos(glasma_ctx* ctx, const double* dev_soa, double* host_with_ghosts, int R, int NP = -1, int p0 = 0);
+// the process's contexts, for the transfers' pinned buffers (transfer.hip)
+void stage_context_created();
+void stage_context_destroyed();
 void host_sync_ghosts(const glasma_ctx* ctx, double* h, int R);
 __global__ void k_set_identity(double* __restrict__ U, long S, int nmat);
 
