@@ -17,21 +17,17 @@ constexpr int kAdjBlock = 256;
 inline dim3 agrid(long n) { return dim3((unsigned)((n + kAdjBlock - 1) / kAdjBlock)); }
 
 // Block order of the backward passes.  nd directions per site block (1, or 3 for the staple passes, which give each
-// thread one link direction); block b runs on XCD b % 8.  With the site blocks a multiple of 8, XCD k takes site
-// blocks [k nsb/8, (k+1) nsb/8) and, for each, its nd directions in turn: a site's y and z neighbours (a row and a
-// plane away) are then read by the same XCD at about the same time, and the three directions of a pass share them in
-// its L2.  In dispatch order (all sites of direction 0, then 1, then 2) the staple gather read 7 times its
-// compulsory bytes from beyond L2.  Otherwise the directions still alternate, without the XCD ranges.
+// thread one link direction); block b runs on XCD b % 8.  XCD k takes the k-th eighth of the (site block, direction)
+// units, a block's directions in turn: a site's y and z neighbours (a row and a plane away) are then read by the same
+// XCD at about the same time, and the three directions of a pass share them in its L2.  In dispatch order (all sites of
+// direction 0, then 1, then 2) the staple gather read 7 times its compulsory bytes from beyond L2.  Lattices whose site
+// blocks are no multiple of 8 once took the directions in turn without the ranges: the gradient over 100 steps took
+// 67.4 ms at 50 x 45 x 100 and 37.2 ms at 33 x 40 x 90, with the ranges 62.8 and 34.6 ms.
 __device__ __forceinline__ void adj_block(long nsb, int nd, long& sb, int& dir) {
-    const long b = blockIdx.x;
-    if (nsb % 8 == 0) {
-        const long i = b >> 3;
-        dir = (int)(i % nd);
-        sb = (b & 7) * (nsb >> 3) + i / nd;
-    } else {
-        dir = (int)(b % nd);
-        sb = b / nd;
-    }
+    const unsigned n = (unsigned)(nsb * nd), k = blockIdx.x % kXcds, i = blockIdx.x / kXcds, r = n % kXcds;
+    const unsigned u = k * (n / kXcds) + (k < r ? k : r) + i;
+    dir = (int)(u % (unsigned)nd);
+    sb = u / (unsigned)nd;
 }
 inline dim3 adj_grid(long n, int nd) { return dim3((unsigned)(nd * ((n + kAdjBlock - 1) / kAdjBlock))); }
 
