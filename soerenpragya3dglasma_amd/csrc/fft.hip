@@ -452,6 +452,19 @@ int fft_fail_hip(hipError_t e, const std::string& what) { return fft_fail(hip_co
 const char* fft_last_error() { return g_fft_err.c_str(); }
 
 hipError_t fft_twiddles(int n, const dbl2** out) { return twiddles(n, out); }
+hipError_t fft_twiddles_split(int n, const dbl2** out) { return twiddles_split(n, out); }
+hipError_t fft_lds_limit(size_t* out) {
+    FftDevice d;
+    const hipError_t e = fft_device(&d);
+    if (e == hipSuccess) *out = d.lds;
+    return e;
+}
+int fft_radices(int n, Radices& R) {
+    if (n > kFftLds) return fft_fail(GLASMA_ERR_ARG, "length " + std::to_string(n) + " is above 2048");
+    if (factorize(n, R) != 0)
+        return fft_fail(GLASMA_ERR_ARG, "length " + std::to_string(n) + " has a prime factor above 13");
+    return 0;
+}
 
 namespace {
 
@@ -972,10 +985,9 @@ int fft_lines_filtered(hipStream_t st, double* data, int n, long es, long nlines
                        const LineFilter& filt) {
     if (n <= 1 || nlines <= 0) return 0;
     if (filt.on && es == 1) return fft_fail(GLASMA_ERR_ARG, "a filtered pass needs strided lines");
-    if (n > kFftLds) return fft_fail(GLASMA_ERR_ARG, "length " + std::to_string(n) + " is above 2048");
     Radices R;
-    if (factorize(n, R) != 0)
-        return fft_fail(GLASMA_ERR_ARG, "length " + std::to_string(n) + " has a prime factor above 13");
+    const int rr = fft_radices(n, R);
+    if (rr) return rr;
     const dbl2* tw = nullptr;
     const hipError_t te = filt.on ? twiddles_split(n, &tw) : twiddles(n, &tw);
     if (te != hipSuccess) return fft_fail_hip(te, "twiddle table");

@@ -69,6 +69,13 @@ __device__ __forceinline__ int qdiv(int a, int d, float rd) {
 
 // the forward twiddle table exp(-2 pi i j / n), j < n, of the current device (fft.hip; kept for the process lifetime)
 hipError_t fft_twiddles(int n, const dbl2** out);
+// the two-level table of twid_split, the same way
+hipError_t fft_twiddles_split(int n, const dbl2** out);
+// the factorisation of a line of length n with the refusals of every transform here (above 2048, a prime factor above
+// 13: an error code, the reason in fft_last_error)
+int fft_radices(int n, Radices& R);
+// LDS a workgroup may ask for on the current device (160 KiB on gfx950 where the runtime grants it)
+hipError_t fft_lds_limit(size_t* out);
 // entries of the two-level table of twid_split
 __host__ __device__ inline int split_entries(int n) { return kTwSplit + (n + kTwSplit - 1) / kTwSplit; }
 
@@ -76,10 +83,10 @@ __host__ __device__ inline int split_entries(int n) { return kTwSplit + (n + kTw
 // lb + c * bs.  Returns which buffer holds the transform.  The buffers are addressed as offsets from the LDS base, not through
 // a run-time indexed pointer array, so the compiler keeps them in the LDS address space (ds_read / ds_write);
 // a generic pointer would give flat instructions, whose waits also wait for every global load in flight.
-// transform.  Every stage ends with a barrier.
+// Every stage ends with a barrier.  Elements of a line lie es apart.
 template <bool SPLIT = false>
 __device__ __forceinline__ int stockham(dbl2* const lb, int bs, int cur, const Radices& R, int lpb, int ld,
-                                        int sign, const dbl2* tw) {
+                                        int sign, const dbl2* tw, int es = 1) {
     const int n = R.n;
     int Ns = 1;
     for (int st = 0; st < R.nst; st++) {
@@ -98,7 +105,7 @@ __device__ __forceinline__ int stockham(dbl2* const lb, int bs, int cur, const R
             dbl2* bl = b + li * ld;
             const int od = jq * Ns * r + k;
             if (r == 4) {
-                dbl2 v0 = al[j], v1 = al[j + nr], v2 = al[j + 2 * nr], v3 = al[j + 3 * nr];
+                dbl2 v0 = al[j * es], v1 = al[(j + nr) * es], v2 = al[(j + 2 * nr) * es], v3 = al[(j + 3 * nr) * es];
                 if (k) {
                     v1 = cmul(v1, twiddle<SPLIT>(tw, k * tstride, sign));
                     v2 = cmul(v2, twiddle<SPLIT>(tw, 2 * k * tstride, sign));
@@ -107,17 +114,17 @@ __device__ __forceinline__ int stockham(dbl2* const lb, int bs, int cur, const R
                 dbl2 t0 = v0 + v2, t1 = v0 - v2, t2 = v1 + v3, d = v1 - v3;
                 // t3 = (sign * i) * d
                 dbl2 t3 = sign < 0 ? dbl2{d.y, -d.x} : dbl2{-d.y, d.x};
-                bl[od] = t0 + t2;
-                bl[od + Ns] = t1 + t3;
-                bl[od + 2 * Ns] = t0 - t2;
-                bl[od + 3 * Ns] = t1 - t3;
+                bl[od * es] = t0 + t2;
+                bl[(od + Ns) * es] = t1 + t3;
+                bl[(od + 2 * Ns) * es] = t0 - t2;
+                bl[(od + 3 * Ns) * es] = t1 - t3;
             } else if (r == 2) {
-                dbl2 v0 = al[j], v1 = al[j + nr];
+                dbl2 v0 = al[j * es], v1 = al[(j + nr) * es];
                 if (k) v1 = cmul(v1, twiddle<SPLIT>(tw, k * tstride, sign));
-                bl[od] = v0 + v1;
-                bl[od + Ns] = v0 - v1;
+                bl[od * es] = v0 + v1;
+                bl[(od + Ns) * es] = v0 - v1;
             } else if (r == 3) {
-                dbl2 v0 = al[j], v1 = al[j + nr], v2 = al[j + 2 * nr];
+                dbl2 v0 = al[j * es], v1 = al[(j + nr) * es], v2 = al[(j + 2 * nr) * es];
                 if (k) {
                     v1 = cmul(v1, twiddle<SPLIT>(tw, k * tstride, sign));
                     v2 = cmul(v2, twiddle<SPLIT>(tw, 2 * k * tstride, sign));
@@ -127,20 +134,20 @@ __device__ __forceinline__ int stockham(dbl2* const lb, int bs, int cur, const R
                 dbl2 m = v0 - 0.5 * t;
                 // (sign * i * h) * d
                 dbl2 q = sign < 0 ? dbl2{h * d.y, -h * d.x} : dbl2{-h * d.y, h * d.x};
-                bl[od] = v0 + t;
-                bl[od + Ns] = m + q;
-                bl[od + 2 * Ns] = m - q;
+                bl[od * es] = v0 + t;
+                bl[(od + Ns) * es] = m + q;
+                bl[(od + 2 * Ns) * es] = m - q;
             } else {
                 // a direct DFT of prime length r <= 13; the inputs are re-read from LDS for each output rather than
                 // held in a run-time indexed array (which would live in scratch memory)
                 for (int p = 0; p < r; p++) {
-                    dbl2 s = al[j];
+                    dbl2 s = al[j * es];
                     for (int q = 1; q < r; q++) {
-                        dbl2 v = al[j + q * nr];
+                        dbl2 v = al[(j + q * nr) * es];
                         if (k) v = cmul(v, twiddle<SPLIT>(tw, (k * q * tstride) % n, sign));
                         s += cmul(v, twiddle<SPLIT>(tw, ((p * q) % r) * nr, sign));
                     }
-                    bl[od + p * Ns] = s;
+                    bl[(od + p * Ns) * es] = s;
                 }
             }
         }

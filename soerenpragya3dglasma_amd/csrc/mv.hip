@@ -22,6 +22,7 @@
 
 #include "internal.h"
 #include "adjoint.h"
+#include "fft_lds.h"
 
 namespace glasma {
 
@@ -32,7 +33,6 @@ struct Wk {
     double* rho = nullptr;
     double* V = nullptr;
     double* xi = nullptr;
-    double* prof = nullptr;  // z profiles of a separable charge (mv_sheet): 4 nz doubles
 };
 
 __device__ __forceinline__ long fidx(const Geom& g, int a, long s) {
@@ -175,109 +175,235 @@ __global__ void k_evolve_phase(double* __restrict__ F, Geom g, double az, double
     }
 }
 
-// The momentum-space factor of mv_sheet over one transverse round trip: smoothing x Poisson,
-// nf exp(-p^2/2 Lambda^2) p^2/(p^2+m^2) / p^2 with the zero mode set to 0, and with `evolve` the z phase of
-// k_evolve_phase (1/Nz included).  F holds the transverse (and, with `evolve`, the z) transform of the charge.
-__global__ void k_sheet_filter(double* __restrict__ F, Geom g, double ax, double ay, double az, double lam, double meff,
-                               double dt, int right, int evolve) {
-    long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.S) return;
-    const int pz = (int)(s / g.P);
-    const long s2 = s - (long)pz * g.P;
-    const int px = (int)(s2 % g.nx), py = (int)(s2 / g.nx);
+// One sheet (nucleus) of an initial state: its direction, the z range [zlo, zhi] of its fields, the plane groups of J
+// that take its J-stat and J, and, for the separable MV charge, the factors of c(z).
+struct SheetSide {
+    int right, zlo, zhi, wstat, wj;
+    int center;
+    double width, mult_norm;
+};
+struct SheetSides {
+    SheetSide s[2];
+    int n;
+};
+SheetSide sheet_side(bool right, int zlo, int zhi, int wstat, int wj) {
+    return SheetSide{right ? 1 : 0, zlo, zhi, wstat, wj, 0, 1.0, 0.0};
+}
+
+// The separable MV charge rho(x, y, z) = c(z) xi(x, y).  Its work array, for n sides with two colours to a complex
+// entry (the filters are real and even in p, so they act on the real and the imaginary part alike):
+//   A    [side][pair][P] complex: xi on the way in, then the potential's transverse factor a(x, y)
+//   prof [side][5 nz]: the evolved transform of c (2 nz), c evolved by dt (nz), and the partial sums of c and of c
+//        evolved from the side the scan starts on up to and including z (nz each)
+__device__ __forceinline__ double mv_profile(const SheetSide& sd, int z) {
+    const double u = (z - sd.center) / sd.width;
+    return sd.mult_norm * (exp(-0.5 * u * u) / sqrt(2.0 * kPi * sd.width * sd.width));  // k_charge's factor
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+// smoothing x Poisson over one transverse round trip: nf exp(-p^2/2 Lambda^2) p^2/(p^2+m^2) / p^2, the zero mode 0
+__device__ __forceinline__ double sheet_filter(const Geom& g, int px, int py, double ax, double ay, double lam,
+                                               double meff) {
+    if (px == 0 && py == 0) return 0.0;
     const double p2 = psqr2(g, px, py, ax, ay);
     const double nf = 1.0 / ((double)g.nx * g.ny);
     const double fs = nf * exp(-p2 / (2.0 * lam * lam)) * p2 / (p2 + meff * meff);
-    const double f = (px == 0 && py == 0) ? 0.0 : fs / p2;
-    double cs = f, sn = 0.0;
-    if (evolve) {
-        const double om = sqrt((2.0 - 2.0 * cos(2.0 * kPi * (double)pz / (double)g.nz)) / (az * az));
-        double sgn;
-        if (!right) sgn = (pz < g.nz / 2) ? -1.0 : 1.0;
-        else sgn = (pz < g.nz / 2) ? 1.0 : -1.0;
-        sincos(sgn * om * dt, &sn, &cs);
-        cs *= f / g.nz;
-        sn *= f / g.nz;
-    }
-    for (int a = 0; a < 8; a++) {
-        const long i = fidx(g, a, s);
-        const double re = F[2 * i], im = F[2 * i + 1];
-        F[2 * i] = cs * re - sn * im;
-        F[2 * i + 1] = sn * re + cs * im;
-    }
+    return fs / p2;
 }
 
-// one transverse slice of F (complex, component-major: entry (a, s2) at a P + s2) = (xi, 0)
-__global__ void k_load_xi(double* __restrict__ F, const double* __restrict__ xi, long P) {
-    const long s2 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s2 >= P) return;
-    for (int a = 0; a < 8; a++) {
-        F[2 * (a * P + s2)] = xi[a + 8 * s2];
-        F[2 * (a * P + s2) + 1] = 0.0;
-    }
-}
-
-// z profiles of the separable MV charge rho(x, y, z) = c(z) xi(x, y): prof[z] = c(z), k_charge's factor; then
-// prof[2 nz + 2 pz (+1)] = sum_z c(z) e^{-2 pi i pz z / nz}, and prof[nz + z] = the real part of the inverse transform
-// of that times k_evolve_phase's factor (the profile evolved by dt).  Direct sums (nz^2 terms), one thread per output.
-__global__ void k_profile_c(double* __restrict__ prof, Geom g, double mult_norm, int center, double width) {
-    const int z = blockIdx.x * blockDim.x + threadIdx.x;
-    if (z >= g.nz) return;
-    const double u = (z - center) / width;
-    prof[z] = mult_norm * (exp(-0.5 * u * u) / sqrt(2.0 * kPi * width * width));
-}
-__global__ void k_profile_dft(double* __restrict__ prof, Geom g) {
-    const int pz = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pz >= g.nz) return;
+// coefficient pz of the side's profile evolved by dt: sum_z c(z) e^{-2 pi i pz z / nz} times k_evolve_phase's factor.
+// One wave per output; the terms are dealt to the lanes.
+__device__ __forceinline__ void profile_dft(double* __restrict__ prof, const SheetSide& sd, int nz, int pz, double az,
+                                            double dt) {
+    const int lane = threadIdx.x & 63;
     double re = 0.0, im = 0.0;
-    for (int z = 0; z < g.nz; z++) {
+    for (int z = lane; z < nz; z += 64) {
         double sn, cs;
-        sincos(-2.0 * kPi * (double)(((long)pz * z) % g.nz) / (double)g.nz, &sn, &cs);
-        re = fma(prof[z], cs, re);
-        im = fma(prof[z], sn, im);
+        sincos(-2.0 * kPi * (double)(((unsigned)pz * (unsigned)z) % (unsigned)nz) / (double)nz, &sn, &cs);
+        const double c = mv_profile(sd, z);
+        re = fma(c, cs, re);
+        im = fma(c, sn, im);
     }
-    prof[2 * g.nz + 2 * pz] = re;
-    prof[2 * g.nz + 2 * pz + 1] = im;
-}
-__global__ void k_profile_evolve(double* __restrict__ prof, Geom g, double az, double dt, int right) {
-    const int z = blockIdx.x * blockDim.x + threadIdx.x;
-    if (z >= g.nz) return;
-    double acc = 0.0;
-    for (int pz = 0; pz < g.nz; pz++) {
-        const double om = sqrt((2.0 - 2.0 * cos(2.0 * kPi * (double)pz / (double)g.nz)) / (az * az));
-        double sgn;
-        if (!right) sgn = (pz < g.nz / 2) ? -1.0 : 1.0;
-        else sgn = (pz < g.nz / 2) ? 1.0 : -1.0;
-        double sp, cp, sn, cs;
-        sincos(sgn * om * dt, &sp, &cp);
-        sincos(2.0 * kPi * (double)(((long)pz * z) % g.nz) / (double)g.nz, &sn, &cs);
-        const double re = prof[2 * g.nz + 2 * pz], im = prof[2 * g.nz + 2 * pz + 1];
-        const double er = cp * re - sp * im, ei = sp * re + cp * im;  // evolved coefficient
-        acc += er * cs - ei * sn;                                       // real part of it times e^{+i ...}
+    re = wave_sum(re);
+    im = wave_sum(im);
+    const double om = sqrt((2.0 - 2.0 * cos(2.0 * kPi * (double)pz / (double)nz)) / (az * az));
+    double sgn;
+    if (!sd.right) sgn = (pz < nz / 2) ? -1.0 : 1.0;
+    else sgn = (pz < nz / 2) ? 1.0 : -1.0;
+    double sp, cp;
+    sincos(sgn * om * dt, &sp, &cp);
+    if (lane == 0) {
+        prof[2 * pz] = cp * re - sp * im;
+        prof[2 * pz + 1] = sp * re + cp * im;
     }
-    prof[g.nz + z] = acc / g.nz;
 }
 
-// The path-ordered Wilson lines of k_wilson_scan for a potential separable in z, A(x, y, z) = cz(z) a(x, y), with a
-// in the real parts of one transverse slice of F (entry (a, s2) at a P + s2)
-__global__ void __launch_bounds__(256) k_wilson_scan_sep(const double* __restrict__ F, const double* __restrict__ cz,
-                                                         double* __restrict__ V, Geom g, int right) {
+// Blocks [0, 4 planes): the transverse factor of one pair of colours, xi -> a(x, y), both transforms and the filter in
+// LDS (two buffers of ny rows of ld entries, then the twiddles of nx and ny).  Every further wave: one coefficient of a
+// side's evolved profile.  The two do not depend on each other and each alone leaves the chip nearly empty.
+// What bounds this kernel is the chain of LDS stages of its one block per pair: 11 us at 16 x 16 x 32, where the separate
+// passes (load, 4 transform launches, filter, 3 profile launches, the profiles' sums by one thread per output) took 70 us
+// and their gaps, and 37 us for two nuclei of 64 x 64, where load, transforms and filter took 74 us.
+constexpr int kPlaneThreads = 512;
+__global__ void __launch_bounds__(kPlaneThreads) k_sheet_plane(const double* __restrict__ xi, dbl2* __restrict__ A,
+                                                               double* __restrict__ prof, Geom g, SheetSides sides,
+                                                               int planes, int ld, Radices Rx, Radices Ry,
+                                                               const dbl2* __restrict__ twx,
+                                                               const dbl2* __restrict__ twy, double ax, double ay,
+                                                               double az, double lam, double meff, double dt) {
+    extern __shared__ dbl2 lds[];
+    if ((int)blockIdx.x >= 4 * planes) {
+        const int u = ((int)blockIdx.x - 4 * planes) * (kPlaneThreads / 64) + (int)(threadIdx.x >> 6);
+        if (u >= sides.n * g.nz) return;
+        const int side = u / g.nz;
+        profile_dft(prof + (long)side * 5 * g.nz, sides.s[side], g.nz, u - side * g.nz, az, dt);
+        return;
+    }
+    const int side = blockIdx.x >> 2, pair = blockIdx.x & 3;  // as in A
+    const int P = (int)g.P, bs = g.ny * ld;
+    dbl2* const tx = lds + 2 * bs;
+    dbl2* const ty = tx + g.nx;
+    for (int k = threadIdx.x; k < g.nx; k += kPlaneThreads) tx[k] = twx[k];
+    for (int k = threadIdx.x; k < g.ny; k += kPlaneThreads) ty[k] = twy[k];
+    const double* const src = xi + 8 * g.P * side + 2 * pair;
+    const float rnx = 1.0f / (float)g.nx;
+    for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
+        const int y = qdiv(i, g.nx, rnx);
+        lds[y * ld + i - y * g.nx] = dbl2{src[8 * i], src[8 * i + 1]};
+    }
+    __syncthreads();
+    int cur = stockham(lds, bs, 0, Rx, g.ny, ld, -1, tx);
+    cur = stockham(lds, bs, cur, Ry, g.nx, 1, -1, ty, ld);
+    for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
+        const int y = qdiv(i, g.nx, rnx), x = i - y * g.nx;
+        lds[cur * bs + y * ld + x] *= sheet_filter(g, x, y, ax, ay, lam, meff);
+    }
+    __syncthreads();
+    cur = stockham(lds, bs, cur, Ry, g.nx, 1, +1, ty, ld);
+    cur = stockham(lds, bs, cur, Rx, g.ny, ld, +1, tx);
+    for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
+        const int y = qdiv(i, g.nx, rnx);
+        A[(long)blockIdx.x * g.P + i] = lds[cur * bs + y * ld + i - y * g.nx];
+    }
+}
+
+// the same in separate passes, for planes beyond the LDS: A = xi with two colours to an entry, and the filter
+__global__ void k_sheet_load(const double* __restrict__ xi, dbl2* __restrict__ A, long P, int n) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 4 * P * n) return;
+    const long q = i / P, s2 = i - q * P;
+    const double* const src = xi + 8 * (P * (q >> 2) + s2) + 2 * (q & 3);
+    A[i] = dbl2{src[0], src[1]};
+}
+__global__ void k_sheet_filter(dbl2* __restrict__ A, Geom g, int ncomp, double ax, double ay, double lam, double meff) {
     const long s2 = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s2 >= g.P) return;
-    double a0[8];
-    for (int a = 0; a < 8; a++) a0[a] = F[2 * (a * g.P + s2)];
-    M3 W, X, T;
-    set_unit(W);
-    const double c = (right ? 1.0 : -1.0) / kSqrt2;
-    for (int k = 0; k < g.nz; k++) {
-        const int z = right ? k : g.nz - 1 - k;
-        const double f = cz[z];
-        double col[8];
-        for (int a = 0; a < 8; a++) col[a] = f * a0[a];
-        expi(c, col, X);
-        mul_nn(X, W, T);
-        W = T;
-        stm<long>(V, kGPlanes, 0, s2 + g.P * z, W);
+    const int px = (int)(s2 % g.nx), py = (int)(s2 / g.nx);
+    const double f = sheet_filter(g, px, py, ax, ay, lam, meff);
+    for (int a = 0; a < ncomp; a++) A[a * g.P + s2] *= f;
+}
+
+// c evolved by dt: the real part of the inverse transform of profile_dft's coefficients.  One wave per z of a side.
+__global__ void __launch_bounds__(256) k_profile_evolve(double* __restrict__ prof, int nz, int n) {
+    const int u = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (u >= n * nz) return;
+    const int side = u / nz, z = u - side * nz;
+    double* const pr = prof + (long)side * 5 * nz;
+    double acc = 0.0;
+    for (int pz = lane; pz < nz; pz += 64) {
+        double sn, cs;
+        sincos(2.0 * kPi * (double)(((unsigned)pz * (unsigned)z) % (unsigned)nz) / (double)nz, &sn, &cs);
+        acc += pr[2 * pz] * cs - pr[2 * pz + 1] * sn;
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) pr[2 * nz + z] = acc / nz;
+}
+// partial sums of c and c evolved in the order of the Wilson lines (left sheet: from Nz - 1 down, right: from 0 up).
+// One block per side: each thread sums a run, the runs' sums are scanned in LDS.
+__global__ void __launch_bounds__(256) k_profile_sums(double* __restrict__ prof, int nz, SheetSides sides) {
+    __shared__ double part[2][2][256];
+    const SheetSide sd = sides.s[blockIdx.x];
+    double* const pr = prof + (long)blockIdx.x * 5 * nz;
+    const int t = threadIdx.x, m = (nz + 255) / 256, k0 = min(nz, t * m), k1 = min(nz, k0 + m);
+    double s0 = 0.0, s1 = 0.0;
+    for (int k = k0; k < k1; k++) {
+        const int z = sd.right ? k : nz - 1 - k;
+        s0 += mv_profile(sd, z);
+        s1 += pr[2 * nz + z];
+    }
+    int b = 0;
+    part[0][0][t] = s0;
+    part[0][1][t] = s1;
+    __syncthreads();
+    for (int o = 1; o < 256; o <<= 1, b ^= 1) {
+        part[b ^ 1][0][t] = part[b][0][t] + (t >= o ? part[b][0][t - o] : 0.0);
+        part[b ^ 1][1][t] = part[b][1][t] + (t >= o ? part[b][1][t - o] : 0.0);
+        __syncthreads();
+    }
+    s0 = t ? part[b][0][t - 1] : 0.0;
+    s1 = t ? part[b][1][t - 1] : 0.0;
+    for (int k = k0; k < k1; k++) {
+        const int z = sd.right ? k : nz - 1 - k;
+        s0 += mv_profile(sd, z);
+        s1 += pr[2 * nz + z];
+        pr[3 * nz + z] = s0;
+        pr[4 * nz + z] = s1;
+    }
+}
+
+// The sheet's U(t + dt), UOld and E(t + dt/2) from the separable potentials A0 = c(z) a(x, y) and A1 = c_ev(z) a(x, y).
+// The exponents of one transverse site along z are multiples of one matrix a(x, y) and commute, so the path-ordered
+// product of SetNewWilsonLines is one exponential, V(z) = exp(+-i a(x, y) / sqrt 2 * sum of c over the layers passed):
+// no serial chain in z, and no Wilson line is stored; each thread forms the four lines its link and its logarithm need.
+// One thread per site and transverse direction (blockIdx.y = 2 side + mu).  Bound by the exponentials and the Jacobi
+// sweeps of the logarithm.  The scans (one thread per transverse site walking z), the link passes and the E pass it
+// replaces took 97 us at 16 x 16 x 32 (60 of them the scans' serial chain), where this takes 23, and for two nuclei
+// 1490 us at 64 x 64 x 256 (534) and 22.2 ms at 256 x 256 x 512 (18.1).
+__global__ void __launch_bounds__(256) k_sheet_sep(const dbl2* __restrict__ A, const double* __restrict__ prof,
+                                                   double* __restrict__ U, double* __restrict__ UO,
+                                                   double* __restrict__ E, Geom g, SheetSides sides, double coff0,
+                                                   double coff1) {
+    const int side = blockIdx.y >> 1, mu = blockIdx.y & 1;
+    const SheetSide& sd = sides.s[side];
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (long)(sd.zhi - sd.zlo + 1) * g.P) return;
+    const long s = i + (long)sd.zlo * g.P;
+    const int z = (int)(s / g.P);
+    const long s2 = s - (long)z * g.P;
+    const int x = (int)(s2 % g.nx), y = (int)(s2 / g.nx);
+    const long sn = mu == 0 ? sidx(g, x + 1, y, 0) : sidx(g, x, y + 1, 0);
+    const dbl2* const Ap = A + 4 * g.P * side;
+    double a[8], b[8];
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const dbl2 v = Ap[p * g.P + s2], w = Ap[p * g.P + sn];
+        a[2 * p] = v.x;
+        a[2 * p + 1] = v.y;
+        b[2 * p] = w.x;
+        b[2 * p + 1] = w.y;
+    }
+    const double* const sums = prof + (long)side * 5 * g.nz + 3 * g.nz;
+    const double c = (sd.right ? 1.0 : -1.0) / kSqrt2;
+    M3 V, W, L[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const double f = c * sums[t * g.nz + z];
+        expi(f, a, V);
+        expi(f, b, W);
+        mul_dn(V, W, L[t]);
+        stm<long>(t ? U : UO, kUPlanes, 18 * mu, s, L[t]);
+    }
+    set_unit(V);
+    stm<long>(mu == 0 ? U : UO, kUPlanes, 36, s, V);
+    mul_nd(L[1], L[0], V);
+    double e[8];
+    ilog(mu == 0 ? coff0 : coff1, V, e);
+    stv<long>(E, kEPlanes, 8 * mu, s, e);
+    if (mu == 0) {
+        double zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        stv<long>(E, kEPlanes, 16, s, zero);
     }
 }
 
@@ -302,9 +428,10 @@ __global__ void __launch_bounds__(256) k_sheet_efield(const double* __restrict__
 }
 
 // J_stat = sqrt2 * sum_{i=x,y} (E_i(x) - U_i^dag(x-i) E_i(x-i) U_i(x-i)) inside [zlo, zhi], 0 outside
-// (:98-125); also F = (J_stat, 0) for the continuity inversion.
-__global__ void __launch_bounds__(256) k_sheet_jstat(const double* __restrict__ U, const double* __restrict__ E, double* __restrict__ J,
-                              double* __restrict__ F, Geom g, int zlo, int zhi, int wstat) {
+// (:98-125), of the side blockIdx.y.
+__global__ void __launch_bounds__(256) k_sheet_jstat(const double* __restrict__ U, const double* __restrict__ E,
+                                                     double* __restrict__ J, Geom g, SheetSides A) {
+    const int zlo = A.s[blockIdx.y].zlo, zhi = A.s[blockIdx.y].zhi, wstat = A.s[blockIdx.y].wstat;
     long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= g.S) return;
     const int z = (int)(s / g.P);
@@ -329,11 +456,6 @@ __global__ void __launch_bounds__(256) k_sheet_jstat(const double* __restrict__ 
         for (int a = 0; a < 8; a++) js[a] = 0.0;
     }
     stv<long>(J, kJPlanes, 8 * wstat, s, js);
-    for (int a = 0; a < 8; a++) {
-        const long i = fidx(g, a, s);
-        F[2 * i] = js[a];
-        F[2 * i + 1] = 0.0;
-    }
 }
 
 // continuity inversion in z momentum space (:131-209):
@@ -387,13 +509,78 @@ __global__ void k_jinv(double* __restrict__ F, Geom g, double az, double dt, int
     }
 }
 
-// J = Re F into planes 8*w of the current-density field
-__global__ void k_store_j(const double* __restrict__ F, double* __restrict__ J, Geom g, int w) {
-    long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.S) return;
-    double v[8];
-    for (int a = 0; a < 8; a++) v[a] = F[2 * fidx(g, a, s)];
-    stv<long>(J, kJPlanes, 8 * w, s, v);
+// factor pz of k_jinv, 1/Nz included
+__device__ __forceinline__ dbl2 jinv_factor(int pz, int nz, double az, double dt, int right) {
+    const double nf = 1.0 / nz;
+    if (pz == 0) return dbl2{nf, 0.0};
+    if (pz == nz / 2) return dbl2{0.0, 0.0};
+    const double om = sqrt((2.0 - 2.0 * cos(2.0 * kPi * (double)pz / (double)nz)) / (az * az));
+    double es, ec, sp, cp;
+    sincos(-2.0 * kPi * (double)pz / (double)nz, &es, &ec);
+    sincos(om * dt, &sp, &cp);
+    // the two branches of k_jinv: e^{+i om dt} - 1 for the lower half of the right sheet's spectrum and the upper
+    // half of the left's, its conjugate otherwise
+    const double mr = cp - 1.0, mi = (right != 0) == (pz < nz / 2) ? sp : -sp;
+    const double sg = right ? 1.0 : -1.0;
+    const double dr = dt * (sg * (1.0 - ec) / az), di = dt * (-sg * es / az);
+    const double den = dr * dr + di * di;
+    return dbl2{nf * ((mr * dr + mi * di) / den), nf * ((mi * dr - mr * di) / den)};
+}
+
+// J from J-stat: the continuity inversion (k_jinv between a forward and an inverse z transform, the real part kept) in
+// one pass over the current field.  A tiled plane pair holds colours 2p and 2p + 1 of a site side by side, so a z line
+// of a pair is read as one complex line: the map takes real lines to real lines once its factors are made Hermitian,
+// h(k) = (H(k) + conj H(Nz - k)) / 2, which is what keeping the real part does.  blockIdx.y = side; a side's lines are
+// taken lpb neighbours at a time by walking blocks, XCD k owning the k-th eighth of the groups.
+// LDS: two buffers of lpb * ld entries, the two-level twiddles, h(k) for k <= Nz / 2.
+// Separate passes (J-stat copied to a complex array, transform, factors, transform, real parts to J) moved 960 bytes a
+// site beyond the J-stat itself; this one moves 128.  Two nuclei at 64 x 64 x 256: 318 us before, 147 now; at
+// 256 x 256 x 512 12.6 and 6.4 ms (the LDS stages; the bytes alone would take 1.4).
+__global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom g, SheetSides sides, Radices R, int lpb,
+                                                    int ld, const dbl2* __restrict__ twg, double az, double dt) {
+    extern __shared__ dbl2 lds[];
+    const int n = R.n, bs = lpb * ld;
+    const SheetSide& sd = sides.s[blockIdx.y];
+    dbl2* const tw = lds + 2 * bs;
+    dbl2* const h = tw + split_entries(n);
+    for (int k = threadIdx.x; k < split_entries(n); k += 256) tw[k] = twg[k];
+    for (int k = threadIdx.x; k <= n / 2; k += 256) {
+        const dbl2 a = jinv_factor(k, n, az, dt, sd.right);
+        const dbl2 b = k ? jinv_factor(n - k, n, az, dt, sd.right) : a;
+        h[k] = dbl2{0.5 * (a.x + b.x), 0.5 * (a.y - b.y)};
+    }
+    const int lg = __builtin_ctz(lpb);
+    const long gpp = (g.P + lpb - 1) / lpb, groups = 4 * gpp;  // groups of a pair, and of the side
+    const long per = (groups + 7) / 8, last = min(groups, (long)(blockIdx.x % 8 + 1) * per);
+    for (long q = (blockIdx.x % 8) * per + blockIdx.x / 8; q < last; q += gridDim.x / 8) {
+        const int pair = (int)(q / gpp);
+        const long s0 = (q - pair * gpp) * lpb;
+        for (int i = threadIdx.x; i < lpb * n; i += 256) {
+            const int li = i & (lpb - 1), z = i >> lg;
+            const long s2 = s0 + li;
+            dbl2 v = dbl2{0.0, 0.0};
+            if (s2 < g.P) v = ld2(J + lidx<long>(kJPlanes, 8 * sd.wstat + 2 * pair, s2 + g.P * z));
+            lds[li * ld + z] = v;
+        }
+        __syncthreads();
+        int cur = stockham<true>(lds, bs, 0, R, lpb, ld, -1, tw);
+        for (int i = threadIdx.x; i < lpb * n; i += 256) {
+            const int li = i & (lpb - 1), k = i >> lg;
+            dbl2 f = h[2 * k <= n ? k : n - k];
+            if (2 * k > n) f.y = -f.y;
+            dbl2* const at = lds + cur * bs + li * ld + k;
+            *at = cmul(f, *at);
+        }
+        __syncthreads();
+        cur = stockham<true>(lds, bs, cur, R, lpb, ld, +1, tw);
+        for (int i = threadIdx.x; i < lpb * n; i += 256) {
+            const int li = i & (lpb - 1), z = i >> lg;
+            const long s2 = s0 + li;
+            const dbl2 v = lds[cur * bs + li * ld + z];
+            if (s2 < g.P) *(dbl2*)(J + lidx<long>(kJPlanes, 8 * sd.wj + 2 * pair, s2 + g.P * z)) = v;
+        }
+        __syncthreads();
+    }
 }
 
 // rho (real, a*S + s) -> host AoS with ghosts (a + 8*Index3D)
@@ -415,14 +602,12 @@ int alloc_work(glasma_ctx* ctx, Wk& w) {
     GL_HIP(ctx, hipMalloc(&w.rho, 8 * (size_t)S * sizeof(double)));
     GL_HIP(ctx, hipMalloc(&w.V, (size_t)kGPlanes * Sp * sizeof(double)));
     GL_HIP(ctx, hipMalloc(&w.xi, 8 * (size_t)ctx->g.P * sizeof(double)));
-    GL_HIP(ctx, hipMalloc(&w.prof, 4 * (size_t)ctx->g.nz * sizeof(double)));
     return 0;
 }
 void free_work(Wk& w) {
     if (w.rho) (void)hipFree(w.rho);
     if (w.V) (void)hipFree(w.V);
     if (w.xi) (void)hipFree(w.xi);
-    if (w.prof) (void)hipFree(w.prof);
     w = Wk();
 }
 
@@ -475,6 +660,38 @@ int set_wilson_lines(glasma_ctx* ctx, Wk& w, const glasma_mv_params* mv, const d
     return wilson_from_charge(ctx, w, mv->lambda, mv->m_eff, right);
 }
 
+// J-stat from the transverse Gauss law and J from the z continuity inversion (RevSingleNucleus.cpp:98-209), all sides
+int sheet_currents(glasma_ctx* ctx, const double* U, const double* E, double* J, const SheetSides& A) {
+    const Geom& g = ctx->g;
+    Radices R;
+    GL_FFT(ctx, fft_radices(g.nz, R));
+    const dbl2* tw = nullptr;
+    GL_HIP(ctx, fft_twiddles_split(g.nz, &tw));
+    size_t most = 0;
+    GL_HIP(ctx, fft_lds_limit(&most));
+    // lines per group: 64-byte rows (4) where three workgroups still fit a CU, else fewer.  The initial state took, at
+    // 128 x 128 x 512, 6.5 to 7.2 ms with 2 lines (39 KiB) and 6.8 with 4 (75 KiB); at 128 x 128 x 1024 13.8 ms with 1
+    // or 2 lines (42, 75 KiB) and 15.4 with 4 (one workgroup per CU).  A line of 2048 alone takes 84 KiB.
+    int lpb = 4;
+    auto bytes = [&](int l) {
+        return sizeof(dbl2) * (2 * (size_t)l * (l > 1 ? g.nz + 1 : g.nz) + split_entries(g.nz) + g.nz / 2 + 1);
+    };
+    while (lpb > 1 && bytes(lpb) > 53 * 1024) lpb /= 2;
+    const size_t lds = bytes(lpb);
+    if (lds > most) return set_error(ctx, GLASMA_ERR_ARG, "the current's z line exceeds the LDS");
+    if (lds > 65536)
+        GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sheet_jinv),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_sheet_jstat, dim3(grid1(g.S).x, A.n), dim3(256), 0, ctx->stream, U, E, J, g, A);
+    // blocks: at most 2048 a side, walking; a multiple of 8 for the XCD ranges
+    const long groups = 4 * ((g.P + lpb - 1) / lpb);
+    const unsigned blocks = (unsigned)(8 * std::min<long>(256, (groups + 7) / 8));
+    hipLaunchKernelGGL(k_sheet_jinv, dim3(blocks, A.n), dim3(256), lds, ctx->stream, J, g, A, R, lpb,
+                       lpb > 1 ? g.nz + 1 : g.nz, tw, ctx->p.a[2], ctx->p.dt);
+    GL_HIP(ctx, hipGetLastError());
+    return 0;
+}
+
 // InitialConditions::SingleSheet for one nucleus over [zlo, zhi]; J-stat into plane group wstat, J into w
 int single_sheet(glasma_ctx* ctx, Wk& w, bool right, int zlo, int zhi, int wstat, int wj) {
     const Geom& g = ctx->g;
@@ -501,69 +718,80 @@ int single_sheet(glasma_ctx* ctx, Wk& w, bool right, int zlo, int zhi, int wstat
     hipLaunchKernelGGL(k_sheet_efield, grid1(nsl), dim3(256), 0, ctx->stream, U, ctx->UOld, ctx->E, g, zlo, zhi, coff0,
                        coff1);
     // J-stat from the transverse Gauss law and J from the z continuity inversion (:98-209)
-    hipLaunchKernelGGL(k_sheet_jstat, grid1(g.S), dim3(256), 0, ctx->stream, U, ctx->E, J, w.F, g, zlo, zhi, wstat);
-    GL_FFT(ctx, fft_z(ctx->stream, w.F, g, 8, -1));
-    hipLaunchKernelGGL(k_jinv, grid1(g.S), dim3(256), 0, ctx->stream, w.F, g, ctx->p.a[2], dt, right ? 1 : 0, 0);
-    GL_FFT(ctx, fft_z(ctx->stream, w.F, g, 8, +1));
-    hipLaunchKernelGGL(k_store_j, grid1(g.S), dim3(256), 0, ctx->stream, w.F, J, g, wj);
-    GL_HIP(ctx, hipGetLastError());
-    return 0;
+    SheetSides A;
+    A.n = 1;
+    A.s[0] = sheet_side(right, zlo, zhi, wstat, wj);
+    return sheet_currents(ctx, U, ctx->E, J, A);
 }
 
-// CollidingObjects::SetWilsonLines and InitialConditions::SingleSheet for one MV nucleus, using that its charge is
-// separable, rho(x, y, z) = c(z) xi(x, y) (SetChargeDensities, k_charge).  The reference smooths the charge (a
-// transverse round trip), solves Poisson (another), and for U(t + dt) evolves the smoothed charge along z (a z round
-// trip) and solves Poisson again, taking real parts in between.  Those filters are linear and each acts on one set of
-// axes, so both potentials factor: A0 = c(z) a(x, y) and A1 = c_ev(z) a(x, y), with a = the smoothing x Poisson of xi
-// on one transverse slice (k_sheet_filter) and c_ev = the real part of c evolved by dt (k_profile_*; the filters are
-// real and even in p, so the real parts taken in between are exact up to round-off).  The Wilson lines are scanned
-// from these factors (k_wilson_scan_sep): no transform of the whole lattice.  m_eff = 0 keeps the separate steps
-// (their smoothing factor is 0/0 at p = 0, which the reference's order spreads over the slice).
-int mv_sheet(glasma_ctx* ctx, Wk& w, const glasma_mv_params* mv, const double* xi_host, bool right, int zlo, int zhi,
-             int wstat, int wj) {
+// CollidingObjects::SetWilsonLines and InitialConditions::SingleSheet for the MV nuclei of an initial state, using that
+// the charge is separable, rho(x, y, z) = c(z) xi(x, y) (SetChargeDensities, k_charge).  The reference smooths the
+// charge (a transverse round trip), solves Poisson (another), and for U(t + dt) evolves the smoothed charge along z (a z
+// round trip) and solves Poisson again, taking real parts in between.  Those filters are linear and each acts on one set
+// of axes, so both potentials factor: A0 = c(z) a(x, y) and A1 = c_ev(z) a(x, y), with a = the smoothing x Poisson of xi
+// on one transverse slice and c_ev = the real part of c evolved by dt (the filters are real and even in p, so the real
+// parts taken in between are exact up to round-off).  Links and E follow from these factors site by site
+// (k_sheet_sep): no transform of the whole lattice and no scan in z.  All sides go through each launch together; their
+// z ranges must not overlap.  m_eff = 0 keeps the separate steps (their smoothing factor is 0/0 at p = 0, which the
+// reference's order spreads over the slice).  xi[side]: host arrays of 8 P doubles.
+int mv_sheets(glasma_ctx* ctx, const glasma_mv_params* mv, SheetSides A, const double* const xi[2]) {
     const Geom& g = ctx->g;
     const double dt = ctx->p.dt;
     const double* a = ctx->p.a;
-    GL_HIP(ctx, hipMemcpyAsync(w.xi, xi_host, 8 * (size_t)g.P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     const double norm = std::sqrt(a[0] * a[1]);
-    const double mult = right ? mv->nucleus_r : mv->nucleus_l;
-    const int center = right ? mv->center_r : mv->center_l;
-    const double sigma = right ? mv->sigma_r : mv->sigma_l;
-    const long nsl = (long)(zhi - zlo + 1) * g.P;
-    double* U = ctx->U[ctx->cur];
-    double* J = ctx->J[ctx->cur];
-    // the transverse factor a(x, y) in the first slice of F
-    Geom g1 = g;
-    g1.nz = 1;
-    g1.S = g.P;
-    hipLaunchKernelGGL(k_load_xi, grid1(g.P), dim3(256), 0, ctx->stream, w.F, w.xi, g.P);
-    GL_FFT(ctx, fft_xy(ctx->stream, w.F, g, 8, 1, -1));
-    hipLaunchKernelGGL(k_sheet_filter, grid1(g.P), dim3(256), 0, ctx->stream, w.F, g1, a[0], a[1], a[2], mv->lambda,
-                       mv->m_eff, dt, right ? 1 : 0, 0);
-    GL_FFT(ctx, fft_xy(ctx->stream, w.F, g, 8, 1, +1));
-    // the z profiles c(z) and c_ev(z)
-    hipLaunchKernelGGL(k_profile_c, grid1(g.nz), dim3(256), 0, ctx->stream, w.prof, g, mult * norm, center, sigma);
-    hipLaunchKernelGGL(k_profile_dft, grid1(g.nz), dim3(256), 0, ctx->stream, w.prof, g);
-    hipLaunchKernelGGL(k_profile_evolve, grid1(g.nz), dim3(256), 0, ctx->stream, w.prof, g, a[2], dt, right ? 1 : 0);
-    // U(t + dt) from A1 (SetWilsonLinesForFirstStep, :33-60), UOld from A0 (:14-27)
-    hipLaunchKernelGGL(k_wilson_scan_sep, grid1(g.P), dim3(256), 0, ctx->stream, w.F, w.prof + g.nz, w.V, g,
-                       right ? 1 : 0);
-    hipLaunchKernelGGL(k_sheet_links, grid1(nsl), dim3(256), 0, ctx->stream, w.V, U, g, zlo, zhi);
-    hipLaunchKernelGGL(k_wilson_scan_sep, grid1(g.P), dim3(256), 0, ctx->stream, w.F, w.prof, w.V, g, right ? 1 : 0);
-    hipLaunchKernelGGL(k_sheet_links, grid1(nsl), dim3(256), 0, ctx->stream, w.V, ctx->UOld, g, zlo, zhi);
-    // E(t + dt/2), J-stat and J as single_sheet (:66-209)
+    long nmax = 0;
+    for (int k = 0; k < A.n; k++) {
+        SheetSide& sd = A.s[k];
+        sd.center = sd.right ? mv->center_r : mv->center_l;
+        sd.width = sd.right ? mv->sigma_r : mv->sigma_l;
+        sd.mult_norm = (sd.right ? mv->nucleus_r : mv->nucleus_l) * norm;
+        nmax = std::max(nmax, (long)(sd.zhi - sd.zlo + 1) * g.P);
+    }
+    Radices Rx, Ry, Rz;
+    GL_FFT(ctx, fft_radices(g.nx, Rx));
+    GL_FFT(ctx, fft_radices(g.ny, Ry));
+    GL_FFT(ctx, fft_radices(g.nz, Rz));
+    GL_RC(ensure_fftbuf(ctx, (size_t)A.n * (16 * (size_t)g.P + 5 * (size_t)g.nz)));
+    dbl2* const F = reinterpret_cast<dbl2*>(ctx->fftbuf);
+    double* const dxi = ctx->fftbuf + 8 * g.P * A.n;
+    double* const prof = dxi + 8 * g.P * A.n;
+    for (int k = 0; k < A.n; k++)
+        GL_HIP(ctx, hipMemcpyAsync(dxi + 8 * g.P * k, xi[k], 8 * (size_t)g.P * sizeof(double), hipMemcpyHostToDevice,
+                                   ctx->stream));
+    // the transverse factor a(x, y) of each side: in one launch where a plane fits the LDS twice (up to about 70 x 70),
+    // together with the profiles' transforms; else in separate passes
+    size_t most = 0;
+    GL_HIP(ctx, fft_lds_limit(&most));
+    const int ld = g.nx | 1;
+    const size_t need = sizeof(dbl2) * (2 * (size_t)g.ny * ld + g.nx + g.ny);
+    const bool plane = need <= most;
+    const dbl2 *twx = nullptr, *twy = nullptr;
+    if (plane) {
+        GL_HIP(ctx, fft_twiddles(g.nx, &twx));
+        GL_HIP(ctx, fft_twiddles(g.ny, &twy));
+        if (need > 65536)
+            GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sheet_plane),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
+    }
+    const int planes = plane ? A.n : 0, wpb = kPlaneThreads / 64;
+    hipLaunchKernelGGL(k_sheet_plane, dim3(4 * planes + (A.n * g.nz + wpb - 1) / wpb), dim3(kPlaneThreads),
+                       plane ? need : 0, ctx->stream, dxi, F, prof, g, A, planes, ld, Rx, Ry, twx, twy, a[0], a[1], a[2],
+                       mv->lambda, mv->m_eff, dt);
+    if (!plane) {
+        hipLaunchKernelGGL(k_sheet_load, grid1(4 * g.P * A.n), dim3(256), 0, ctx->stream, dxi, F, g.P, A.n);
+        GL_FFT(ctx, fft_xy(ctx->stream, ctx->fftbuf, g, 4 * A.n, 1, -1));
+        hipLaunchKernelGGL(k_sheet_filter, grid1(g.P), dim3(256), 0, ctx->stream, F, g, 4 * A.n, a[0], a[1], mv->lambda,
+                           mv->m_eff);
+        GL_FFT(ctx, fft_xy(ctx->stream, ctx->fftbuf, g, 4 * A.n, 1, +1));
+    }
+    hipLaunchKernelGGL(k_profile_evolve, dim3((A.n * g.nz + 3) / 4), dim3(256), 0, ctx->stream, prof, g.nz, A.n);
+    hipLaunchKernelGGL(k_profile_sums, dim3(A.n), dim3(256), 0, ctx->stream, prof, g.nz, A);
+    // U(t + dt) from A1 (SetWilsonLinesForFirstStep, :33-60), UOld from A0 (:14-27), E(t + dt/2) (:66-92)
     const double acube = a[0] * a[1] * a[2];
-    const double coff0 = -dt * a[0] * a[0] / acube;
-    const double coff1 = -dt * a[1] * a[1] / acube;
-    hipLaunchKernelGGL(k_sheet_efield, grid1(nsl), dim3(256), 0, ctx->stream, U, ctx->UOld, ctx->E, g, zlo, zhi, coff0,
-                       coff1);
-    hipLaunchKernelGGL(k_sheet_jstat, grid1(g.S), dim3(256), 0, ctx->stream, U, ctx->E, J, w.F, g, zlo, zhi, wstat);
-    GL_FFT(ctx, fft_z(ctx->stream, w.F, g, 8, -1));
-    hipLaunchKernelGGL(k_jinv, grid1(g.S), dim3(256), 0, ctx->stream, w.F, g, a[2], dt, right ? 1 : 0, 0);
-    GL_FFT(ctx, fft_z(ctx->stream, w.F, g, 8, +1));
-    hipLaunchKernelGGL(k_store_j, grid1(g.S), dim3(256), 0, ctx->stream, w.F, J, g, wj);
-    GL_HIP(ctx, hipGetLastError());
-    return 0;
+    double* U = ctx->U[ctx->cur];
+    hipLaunchKernelGGL(k_sheet_sep, dim3(grid1(nmax).x, 2 * A.n), dim3(256), 0, ctx->stream, F, prof, U, ctx->UOld, ctx->E,
+                       g, A, -dt * a[0] * a[0] / acube, -dt * a[1] * a[1] / acube);
+    return sheet_currents(ctx, U, ctx->E, ctx->J[ctx->cur], A);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -930,13 +1158,10 @@ int ic_left_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, const doubl
     const double coff0 = -dt * ctx->p.a[0] * ctx->p.a[0] / acube;
     const double coff1 = -dt * ctx->p.a[1] * ctx->p.a[1] / acube;
     hipLaunchKernelGGL(k_sheet_efield, grid1(g.S), dim3(256), 0, st, U, ctx->UOld, ctx->E, g, 0, g.nz - 1, coff0, coff1);
-    hipLaunchKernelGGL(k_sheet_jstat, grid1(g.S), dim3(256), 0, st, U, ctx->E, J, F, g, 0, g.nz - 1, JPS);
-    GL_FFT(ctx, fft_z(st, F, g, 8, -1));
-    hipLaunchKernelGGL(k_jinv, grid1(g.S), dim3(256), 0, st, F, g, ctx->p.a[2], dt, 0, 0);
-    GL_FFT(ctx, fft_z(st, F, g, 8, +1));
-    hipLaunchKernelGGL(k_store_j, grid1(g.S), dim3(256), 0, st, F, J, g, JP);
-    GL_HIP(ctx, hipGetLastError());
-    return 0;
+    SheetSides A;
+    A.n = 1;
+    A.s[0] = sheet_side(false, 0, g.nz - 1, JPS, JP);
+    return sheet_currents(ctx, U, ctx->E, J, A);
 }
 
 // Reverse-mode derivative of ic_left_from_charge.  In: cotangents of the sheet's U (Ub, tiled 54 planes;
@@ -1038,25 +1263,33 @@ extern "C" int glasma_mv_initial_state(glasma_ctx* ctx, int driver, const glasma
     int rc = reset_for_sheets(ctx, driver);
     if (rc) return rc;
     const int nz = ctx->g.nz;
-    Wk w;
-    rc = alloc_work(ctx, w);
-    if (rc == 0 && driver != 2) {
-        // collision: left sheet on [0, (Nz-2)/2] (SC/Simulation.cpp:359); single nucleus: all z
-        const int zhi = driver == 0 ? (nz - 2) / 2 : nz - 1;
-        if (mv->m_eff > 0.0) {
-            rc = mv_sheet(ctx, w, mv, xi_l, false, 0, zhi, JPS, JP);
-        } else {
-            rc = set_wilson_lines(ctx, w, mv, xi_l, false);
-            if (rc == 0) rc = single_sheet(ctx, w, false, 0, zhi, JPS, JP);
-        }
+    // collision: left sheet on [0, (Nz-2)/2] (SC/Simulation.cpp:359), right on [Nz/2, Nz-1]; single nucleus: all z
+    SheetSides sides;
+    const double* xi[2] = {xi_l, xi_r};
+    sides.n = 0;
+    if (driver != 2) sides.s[sides.n++] = sheet_side(false, 0, driver == 0 ? (nz - 2) / 2 : nz - 1, JPS, JP);
+    if (driver != 1) {
+        xi[sides.n] = xi_r;
+        sides.s[sides.n++] = sheet_side(true, driver == 0 ? nz / 2 : 0, nz - 1, JMS, JM);
     }
-    if (rc == 0 && driver != 1) {
-        const int zlo = driver == 0 ? nz / 2 : 0;
-        if (mv->m_eff > 0.0) {
-            rc = mv_sheet(ctx, w, mv, xi_r, true, zlo, nz - 1, JMS, JM);
+    Wk w;
+    if (mv->m_eff > 0.0) {
+        if (sides.n == 2 && nz == 1) {  // the two ranges overlap: the right sheet after the left
+            SheetSides one;
+            one.n = 1;
+            for (int k = 0; k < 2 && rc == 0; k++) {
+                one.s[0] = sides.s[k];
+                rc = mv_sheets(ctx, mv, one, xi + k);
+            }
         } else {
-            rc = set_wilson_lines(ctx, w, mv, xi_r, true);
-            if (rc == 0) rc = single_sheet(ctx, w, true, zlo, nz - 1, JMS, JM);
+            rc = mv_sheets(ctx, mv, sides, xi);
+        }
+    } else {
+        rc = alloc_work(ctx, w);
+        for (int k = 0; k < sides.n && rc == 0; k++) {
+            const SheetSide& sd = sides.s[k];
+            rc = set_wilson_lines(ctx, w, mv, xi[k], sd.right != 0);
+            if (rc == 0) rc = single_sheet(ctx, w, sd.right != 0, sd.zlo, sd.zhi, sd.wstat, sd.wj);
         }
     }
     if (rc == 0) {
