@@ -17,13 +17,15 @@
 // 1.40x the compulsory bytes (the y-halo rows of a band belong to another XCD, and the tiles in flight
 // outgrow an XCD's 4 MB L2); writes are exactly compulsory.
 //
-// GLASMA_STEP_WAVES (2 or 3: register budget of 256 or 168 per lane) and GLASMA_STEP_MAP / _BW / _BH select variants
-// for measurement sweeps; the defaults are the fastest measured on MI355X.
+// GLASMA_STEP_WAVES (2 or 3: register budget of 256 or 168 per lane, for lattices below 2^32 sites) and
+// GLASMA_STEP_MAP / _BW / _BH select variants for measurement sweeps; the defaults are the fastest measured on MI355X.
 #include <cstdlib>
 
 #include "internal.h"
 
 namespace glasma {
+
+constexpr int kCus = 256;  // compute units of the chip
 
 static int env_int(const char* name, int dflt) {
     const char* v = std::getenv(name);
@@ -389,13 +391,25 @@ StepArgs step_args(const glasma_ctx* ctx, int cur, bool write_old) {
     return A;
 }
 
-template <class I>
-static void launch(int waves, const TileMap& tm, const StepArgs& A, hipStream_t st) {
+template <class I, int W>
+static void launch(const TileMap& tm, const StepArgs& A, hipStream_t st) {
     dim3 grid((unsigned)(pad_sites(A.g.S) / kTile));
-    // three waves per SIMD (168 registers) measured faster than two (30.1 against 31.8 ms at 256 x 256 x 1024)
-    if (row_form(A.g) == 2) hipLaunchKernelGGL((k_step4<I, 3, true>), grid, dim3(256), 0, st, A, tm);
-    else if (waves == 2) hipLaunchKernelGGL((k_step4<I, 2, false>), grid, dim3(256), 0, st, A, tm);
-    else hipLaunchKernelGGL((k_step4<I, 3, false>), grid, dim3(256), 0, st, A, tm);
+    if (row_form(A.g) == 2) hipLaunchKernelGGL((k_step4<I, W, true>), grid, dim3(256), 0, st, A, tm);
+    else hipLaunchKernelGGL((k_step4<I, W, false>), grid, dim3(256), 0, st, A, tm);
+}
+
+// Waves per SIMD of the step, that is workgroups (one tile each) per CU: three with 168 registers or two with 183.
+// Three keep more loads in flight (64 x 64 x 64 0.120 ms against 0.124, 256 x 256 x 1024 30.1 against 31.8).  Two are
+// the better where three have nothing to add: up to two tiles per CU, all resident either way, gain by the registers
+// (256 tiles 11.3 us against 12.5, 512 tiles 18.8 against 19.0), and four per CU run as 2 + 2
+// instead of 3 + 1 (960 tiles 32.6 us against 34.5, 1024 tiles 33.5 against 36.3).  Three per CU are a single round
+// (768 tiles 26.7 us against 29.5), and from five on the tail matters less (1152 tiles 39.4 against 39.6, 1536 tiles
+// 48.5 against 50.0).
+static int step_waves(const Geom& g) {
+    static const int env = env_int("GLASMA_STEP_WAVES", 0);
+    if (env == 2 || env == 3) return env;
+    const long per_cu = (pad_sites(g.S) / kTile + kCus - 1) / kCus;
+    return per_cu <= 2 || per_cu == 4 ? 2 : 3;
 }
 
 // tile order for a geometry: the requested mode when the lattice fits it, else the next simpler one
@@ -453,10 +467,10 @@ TileMap ctx_tile_map(const glasma_ctx* ctx) { return ctx->tm_tuned ? ctx->tm : d
 
 // one step with explicit buffers and tile order (the context supplies the stream)
 int launch_step_map(glasma_ctx* ctx, const StepArgs& A, const TileMap& tm, hipStream_t st) {
-    static const int waves = env_int("GLASMA_STEP_WAVES", 3);
     if (!st) st = ctx->stream;
-    if (A.g.S < (1L << 32)) launch<unsigned int>(waves, tm, A, st);
-    else launch<unsigned long>(waves, tm, A, st);
+    if (A.g.S >= (1L << 32)) launch<unsigned long, 3>(tm, A, st);
+    else if (step_waves(A.g) == 2) launch<unsigned int, 2>(tm, A, st);
+    else launch<unsigned int, 3>(tm, A, st);
     return 0;
 }
 
