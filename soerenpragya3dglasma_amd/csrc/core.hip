@@ -318,23 +318,6 @@ __global__ void __launch_bounds__(256) k_unitarity(ObsArgs A) {
     block_store_max<1>(m, out + 1);
 }
 
-// The same plane of links at several sites, element by element: sites that differ by one in x share their cache lines,
-// which then come once from L2.
-template <int N>
-__device__ __forceinline__ void ld_group(const double* __restrict__ U, int mu, const long (&s)[N], M3 (&M)[N]) {
-    const double* q[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) q[i] = site_ptr<long>(U, kUPlanes, 18 * mu, s[i]);
-#pragma unroll
-    for (int k = 0; k < 9; k++)
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            const d2_t v = ld2(q[i] + k * 2 * kTile);
-            M[i].re[k] = v.x;
-            M[i].im[k] = v.y;
-        }
-}
-
 // Re tr(A B)
 __device__ __forceinline__ double tr_nn(const M3& A, const M3& B) {
     double r = 0.0;
@@ -360,8 +343,8 @@ __device__ __forceinline__ void clover(const double* __restrict__ W, const Geom&
     M3 Y1, Z1, Y, T;
     {
         M3 G[3], H[2], A;
-        ld_group<3>(W, n, {at(0, 0), at(1, 0), at(-1, 0)}, G);
-        ld_group<2>(W, m, {at(0, 1), at(-1, 1)}, H);
+        ld_group<long, 3>(W, kUPlanes, 18 * n, {at(0, 0), at(1, 0), at(-1, 0)}, G);
+        ld_group<long, 2>(W, kUPlanes, 18 * m, {at(0, 1), at(-1, 1)}, H);
         mul_nd(G[1], H[0], A);
         mul_nd(A, G[0], Y1);
         mul_dd(H[1], G[2], A);
@@ -370,15 +353,15 @@ __device__ __forceinline__ void clover(const double* __restrict__ W, const Geom&
     M3 Y2, Z2;
     {
         M3 G[3], H[2], A;
-        ld_group<3>(W, n, {at(0, -1), at(1, -1), at(-1, -1)}, G);
-        ld_group<2>(W, m, {at(0, -1), at(-1, -1)}, H);
+        ld_group<long, 3>(W, kUPlanes, 18 * n, {at(0, -1), at(1, -1), at(-1, -1)}, G);
+        ld_group<long, 2>(W, kUPlanes, 18 * m, {at(0, -1), at(-1, -1)}, H);
         mul_nn(H[0], G[1], A);
         mul_dn(A, G[0], Y2);
         mul_dn(G[2], H[1], A);
         mul_dd(G[0], A, Z2);
     }
     M3 S[2];
-    ld_group<2>(W, m, {at(0, 0), at(-1, 0)}, S);
+    ld_group<long, 2>(W, kUPlanes, 18 * m, {at(0, 0), at(-1, 0)}, S);
     double t = tr_nn(S[0], Y1) + tr_nn(S[0], Y2) + tr_nn(Z1, S[1]) + tr_nn(Z2, S[1]);
 #pragma unroll
     for (int k = 0; k < 9; k++) {

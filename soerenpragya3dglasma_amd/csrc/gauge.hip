@@ -42,6 +42,7 @@ namespace glasma {
 namespace {
 
 constexpr int kCgBlock = 256;
+constexpr long kCgRound = 512;  // blocks of two waves per SIMD that the chip's 256 CUs hold at once
 
 inline dim3 grid1(long n) { return dim3((unsigned)((n + kCgBlock - 1) / kCgBlock)); }
 
@@ -52,9 +53,9 @@ inline dim3 grid1(long n) { return dim3((unsigned)((n + kCgBlock - 1) / kCgBlock
 // one before or after it on the same XCD, its z neighbours h units back or ahead, so both are still in that XCD's
 // L2 (at 256 x 256 x 1024, h = 16 units of links and G are 2.4 MB against 4 MB of L2).  In flat order a unit's y
 // neighbours run on other XCDs and its z neighbours a whole plane (37 MB) apart: the deviation kernel then read
-// 2.5 times its compulsory bytes.  Otherwise (P not a multiple of 256 sites) blocks take units in flat order.
+// 2.5 times its compulsory bytes.  Otherwise (P not a multiple of 256 sites) XCD k takes the k-th eighth of the units.
 struct CgOrder {
-    long upx;  // units per plane per XCD; 0: flat order
+    long upx;  // units per plane per XCD; 0: each XCD an eighth of all units
     int h;     // units per chunk
 };
 
@@ -72,9 +73,15 @@ CgOrder cg_order(const Geom& g) {
     return {U / 8, h};
 }
 
+// Block b runs on XCD b % 8: unit u such that XCD k takes the k-th eighth of the n units, whatever n
+__device__ __forceinline__ unsigned xcd_eighth(unsigned b, unsigned n) {
+    const unsigned k = b % kXcds, r = n % kXcds;
+    return k * (n / kXcds) + (k < r ? k : r) + b / kXcds;
+}
+
 // the first site of this block's unit plus threadIdx.x (callers check s < S for the flat order's last block)
 __device__ __forceinline__ long cg_site(const Geom& g, const CgOrder& o) {
-    if (o.upx == 0) return (long)blockIdx.x * kCgBlock + threadIdx.x;
+    if (o.upx == 0) return (long)xcd_eighth(blockIdx.x, gridDim.x) * kCgBlock + threadIdx.x;
     const long b = blockIdx.x;
     const long k = b & 7, i = b >> 3;
     const long per_chunk = (long)g.nz * o.h;
@@ -255,6 +262,22 @@ __device__ __forceinline__ void w_terms(const double* __restrict__ U, const doub
     }
 }
 
+// G(x) and the direction-x terms (w_terms with mu = 0): the sites x - 1, x and x + 1 share their cache lines, so their
+// matrices are read together and the shared lines come once from L2 (read apart, each matrix's nine kilobytes a wave are
+// gone from the 32 KB L1 before the next)
+__device__ __forceinline__ void w_x(const double* __restrict__ U, const double* __restrict__ G, const Geom& g, long s,
+                                    int x, int y, int z, double c, M3& Gx, double* q) {
+    const long su = sidx(g, x + 1, y, z), sd = sidx(g, x - 1, y, z);
+    M3 Gn[3], Um[2], T;
+    ld_group<long, 3>(G, kGPlanes, 0, {su, sd, s}, Gn);
+    ld_group<long, 2>(U, kUPlanes, 0, {s, sd}, Um);
+    Gx = Gn[2];
+    mul_nn(Gx, Um[0], T);
+    acc_proj_nd(c, T, Gn[0], q);
+    mul_nn(Gn[1], Um[1], T);
+    acc_proj_nd(c, Gx, T, q);
+}
+
 template <bool CONS>
 __device__ __forceinline__ void local_w_fused(const double* __restrict__ U, const double* __restrict__ G,
                                               const double* __restrict__ Gtop, const Geom& g, int x, int y, int z,
@@ -262,11 +285,10 @@ __device__ __forceinline__ void local_w_fused(const double* __restrict__ U, cons
     M3 Gx;
     const double zf = g.nz > 1 ? 1.0 : 0.0;
     const long s = sidx(g, x, y, z);
-    ldm<long>(G, kGPlanes, 0, s, Gx);  // G(x), read once: it starts every forward term and ends every backward one
     for (int k = 0; k < 10; k++) q[k] = 0.0;
+    w_x(U, G, g, s, x, y, z, cx, Gx, q);  // G(x), read once: it starts every forward term and ends every backward one
 #pragma unroll 1
-    for (int mu = 0; mu < 3; mu++)
-        w_terms<CONS>(U, G, Gtop, g, mu, s, x, y, z, mu == 0 ? cx : (mu == 1 ? cy : zf * cz), Gx, q);
+    for (int mu = 1; mu < 3; mu++) w_terms<CONS>(U, G, Gtop, g, mu, s, x, y, z, mu == 1 ? cy : zf * cz, Gx, q);
 }
 
 // Delta^a = Re tr(i t^a w) (retr_igen) from the accumulators of acc_proj_nd
@@ -290,7 +312,7 @@ constexpr int kXfEntries = 4 * kCgBlock;  // complex entries of one LDS buffer: 
 // Delta and the functional (CoulombGaugeDeviation.cpp:23-41, FourierAcceleration.cpp:20-52), with the monitors,
 // from the ungauged links and G.  XF: the four arrays leave x-transformed (R: the factors of Nx, tw: its twiddles).
 template <bool CONS, bool XF>
-__global__ __launch_bounds__(kCgBlock, 3) void k_cg_dev_fused(const double* __restrict__ U, const double* __restrict__ G,
+__global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_fused(const double* __restrict__ U, const double* __restrict__ G,
                                                             const double* __restrict__ Gtop, double* __restrict__ F,
                                                             double* __restrict__ part, Geom g, double cx, double cy,
                                                             double cz, double fm0, CgOrder o, Radices R,
@@ -332,19 +354,18 @@ __global__ __launch_bounds__(kCgBlock, 3) void k_cg_dev_fused(const double* __re
     block_partials(sq, fs, mx, fm, part + 4 * (long)blockIdx.x);
 }
 
-// The deviation kernel walking z (P a multiple of 256): block b takes unit u (sites [256 u, 256 u + 256) of a plane)
+// The deviation kernel walking z: a block takes unit u (sites [256 u, 256 u + 256) of a plane)
 // in the z chunk [z0, z0 + zc) and walks it plane by plane.  The backward z term at z is the adjoint of the forward z
 // term at z - 1, A = U^G_z(z - 1), and the accumulators of A^dag are those of A with the eight anti-Hermitian ones
 // negated and Re tr unchanged: the walk carries those ten numbers from one plane to the next instead of reading
 // G(z - 1) and U_z(z - 1) and forming the link again, and G(z + 1), read for the forward term, is G(x) of the next
 // plane.  That is three matrices read per site less than k_cg_dev_fused, among them the two whose planes lie furthest
-// away.  With XCD order (U = P / 256 units a multiple of 8), XCD k (= b % 8) owns units [k U/8, (k+1) U/8) of every
-// chunk, so the y neighbour units run on the same XCD.  Two waves per SIMD (at three the kernel spills and was slower
-// than k_cg_dev_fused): at 256 x 256 x 1024 the Fourier iteration took 25.2 ms with chunks of 32 planes, 25.6 ms
-// with 16, against 27.1 ms with k_cg_dev_fused.
+// away.  XCD k takes the k-th eighth of the blocks, chunk by chunk: a unit's y neighbours run on the same XCD at the
+// same time.  Two waves per SIMD (at three the kernel spills and was slower than k_cg_dev_fused; reading the sites
+// x - 1, x, x + 1 together, as w_x does, spills at two and gained nothing).  Time goes into the reads' latency.
 struct CgWalk {
-    int zc;   // planes per chunk
-    int xcd;  // XCD order
+    int zc;      // planes per chunk
+    unsigned n;  // blocks: units of a plane x chunks
 };
 
 template <bool CONS, bool XF>
@@ -354,27 +375,18 @@ __global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_walk(const double* __res
                                                            double cz, double fm0, CgWalk o, Radices R,
                                                            const dbl2* __restrict__ tw) {
     __shared__ dbl2 xb[XF ? 2 * kXfEntries : 1];
-    const long nu = g.P / kCgBlock;
-    long unit, zcid;
-    if (o.xcd) {
-        const long b = blockIdx.x, upx = nu / 8;
-        const long i = b >> 3;
-        zcid = i / upx;
-        unit = (b & 7) * upx + (i - zcid * upx);
-    } else {
-        zcid = blockIdx.x / nu;
-        unit = blockIdx.x - zcid * nu;
-    }
+    const unsigned nu = (unsigned)((g.P + kCgBlock - 1) / kCgBlock);
+    const unsigned b = xcd_eighth(blockIdx.x, o.n), zcid = b / nu, unit = b - zcid * nu;
     const int z0 = (int)zcid * o.zc, z1 = min(z0 + o.zc, g.nz);
-    const long s2 = unit * kCgBlock + threadIdx.x;
+    const long s2 = (long)unit * kCgBlock + threadIdx.x;
     const int x = (int)(s2 % g.nx), y = (int)(s2 / g.nx);
     const double czf = g.nz > 1 ? cz : 0.0;
     double sq = 0.0, fs = 0.0, mx = 0.0, fm = fm0;
     M3 Gx;
-    ldm<long>(G, kGPlanes, 0, s2 + (long)z0 * g.P, Gx);
+    if (s2 < g.P) ldm<long>(G, kGPlanes, 0, s2 + (long)z0 * g.P, Gx);
     double pz[10];  // accumulators of the forward z term of the previous plane
 #pragma unroll 1
-    for (int z = z0; z < z1; z++) {
+    for (int z = s2 < g.P ? z0 : z1; z < z1; z++) {  // XF: P is a multiple of 256, every thread walks
         const long s = s2 + (long)z * g.P;
         double q[10];
         for (int k = 0; k < 10; k++) q[k] = 0.0;
@@ -437,23 +449,30 @@ __global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_walk(const double* __res
     block_partials(sq, fs, mx, fm, part + 4 * (long)blockIdx.x);
 }
 
-// the walk where P is a multiple of 256 and chunks of 32 or 16 planes still give 2048 blocks (eight per CU), else
-// k_cg_dev_fused (at 64 x 64 x 256, 1024 blocks of 16 planes, the walk took 0.62 ms per iteration against 0.56);
+// The walk with the longest chunk, of 32, 16, 8 or 4 planes, whose blocks fill rounds of 512 (two per CU) to nine tenths,
+// else k_cg_dev_fused: a longer chunk reads fewer extra planes, but its blocks are long too, and a round that is partly
+// empty costs more than the walk saves.  With the x transforms fused in, every block must be whole (P a multiple of
+// 256).  Deviation kernel, k_cg_dev_fused against the walk with 32, 16, 8 and 4 planes (blocks): 128 x 128 x 256 696 us
+// against 638 (512), 650, 652; 64 x 64 x 256 183 against 307 (128), 177 (256), 167 (512); 125 x 125 x 250 666 against
+// 642 (496); 96 x 96 x 128 197 against 237 (144), 261 (288), 222 (576), 202 (1152); 81 x 75 x 125 127 against 141 with 4
+// (768); 100 x 100 x 100 167 against 165 with 4 (1000); 64 x 64 x 128 92 against 85 with 4 (512).
 // GLASMA_CG_WALK = planes per chunk overrides, 0 turns the walk off
-CgWalk cg_walk(const Geom& g) {
+CgWalk cg_walk(const Geom& g, bool xf) {
     const char* e = std::getenv("GLASMA_CG_WALK");  // read per call, so that tests can set it
     const int forced = e ? std::atoi(e) : -1;
-    if (forced == 0 || g.P % kCgBlock) return {0, 0};
-    const long nu = g.P / kCgBlock;
+    if (forced == 0 || (xf && g.P % kCgBlock)) return {0, 0};
+    const long nu = (g.P + kCgBlock - 1) / kCgBlock;
+    auto blocks = [&](int c) { return nu * ((g.nz + c - 1) / c); };
     int zc = forced > 0 ? forced : 0;
     if (!zc)
-        for (int c : {32, 16})
-            if (nu * ((g.nz + c - 1) / c) >= 2048) {
+        for (int c : {32, 16, 8, 4})
+            if (10 * blocks(c) >= 9 * kCgRound * ((blocks(c) + kCgRound - 1) / kCgRound)) {
                 zc = c;
                 break;
             }
-    if (!zc) return {0, 0};
-    return {zc, nu % 8 == 0 ? 1 : 0};
+    // planes that fill their units to 7/8, and no more blocks than the partials' array has places (one per 256 sites)
+    if (!zc || 8 * g.P < 7 * nu * kCgBlock || blocks(zc) > (g.S + kCgBlock - 1) / kCgBlock) return {0, 0};
+    return {zc, (unsigned)blocks(zc)};
 }
 
 // rows P and Q of X <- A X, A the identity outside the SU(2) block [[a, b], [c, d]] of rows / columns P, Q
@@ -759,14 +778,13 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     const long nblk = (g.S + kCgBlock - 1) / kCgBlock;
     const bool cons = algo == GLASMA_GAUGE_FOURIER_CONSISTENT;
     const CgOrder ord = cg_order(g);
-    const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g);
-    const long nwalk = walk.zc ? g.P / kCgBlock * ((g.nz + walk.zc - 1) / walk.zc) : 0;
     // the x transforms fused into the deviation and update kernels (the Fourier steps with Nz >= 2)
     Radices R{};
     const dbl2* tw = nullptr;
     const bool xf = (algo == GLASMA_GAUGE_FOURIER || cons) && g.nz >= 2 && g.S % kCgBlock == 0 &&
                     kCgBlock % g.nx == 0 && factorize(g.nx, R) == 0 && fft_twiddles(g.nx, &tw) == hipSuccess;
     (void)hipGetLastError();
+    const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g, xf);
     rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + kReduceTmp);
     if (!rc && algo != GLASMA_GAUGE_LOS_ALAMOS) rc = ensure_fftbuf(ctx, 8 * (size_t)g.S);  // 4 complex per site
     if (rc) return rc;
@@ -802,7 +820,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
         } else {
 #define GLASMA_CG_DEV(C, X)                                                                                     \
     if (walk.zc)                                                                                                 \
-        hipLaunchKernelGGL((k_cg_dev_walk<C, X>), dim3((unsigned)nwalk), dim3(kCgBlock), 0, ctx->stream,            \
+        hipLaunchKernelGGL((k_cg_dev_walk<C, X>), dim3(walk.n), dim3(kCgBlock), 0, ctx->stream,            \
                            ctx->U[ctx->cur], ctx->G, ctx->Gtop, F, part, g, cx, cy, cz, fm0, walk, R, tw);         \
     else                                                                                                         \
         hipLaunchKernelGGL((k_cg_dev_fused<C, X>), dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream,           \
@@ -822,7 +840,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
                 hipLaunchKernelGGL(k_cg_sync_top, grid1(g.P), dim3(kCgBlock), 0, ctx->stream, ctx->G, ctx->Gtop, g);
             }
 #undef GLASMA_CG_DEV
-            reduce_partials(ctx->stream, part, walk.zc ? nwalk : nblk, fin, fm0, tmp);
+            reduce_partials(ctx->stream, part, walk.zc ? (long)walk.n : nblk, fin, fm0, tmp);
             if (cons) {
                 // the Laplacian of the links that exist (open z: the Neumann Laplacian, a cosine transform in z); the
                 // zero mode (zero by construction) dropped

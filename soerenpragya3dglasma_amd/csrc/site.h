@@ -136,6 +136,22 @@ GHD void ldm(const double* __restrict__ base, int NP, int p0, I s, M3& A) {
         A.im[k] = v.y;
     }
 }
+// The same matrix of a field at several sites, element by element: sites that differ by one in x share their cache lines,
+// which then come once from L2.
+template <class I, int N>
+GHD void ld_group(const double* __restrict__ base, int NP, int p0, const I (&s)[N], M3 (&A)[N]) {
+    const double* q[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) q[i] = site_ptr<I>(base, NP, p0, s[i]);
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const d2_t v = ld2(q[i] + k * 2 * kTile);
+            A[i].re[k] = v.x;
+            A[i].im[k] = v.y;
+        }
+}
 template <class I>
 GHD void stm(double* __restrict__ base, int NP, int p0, I s, const M3& A) {
     double* q = site_ptr<I>(base, NP, p0, s);
