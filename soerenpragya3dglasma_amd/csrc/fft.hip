@@ -9,9 +9,9 @@
 // neighbouring addresses), runs a self-sorting Stockham transform in LDS (radix 4, 2, 3 kernels, any other
 // prime <= 13 by a direct DFT) and writes the lines back in place.  Multi-dimensional transforms are one pass per
 // axis, so each pass reads and writes the array once.
-// - Strided lines (the y and z passes) go 4 to a group within the device's LDS (160 KiB on gfx950), so each row
-//   of a load is 64 contiguous bytes; their groups are dealt to the XCDs so that neighbouring groups run on one
-//   XCD and share the rest of each 128-byte line in its L2.
+// - Strided lines (the y and z passes) go 4 or more to a group (about 1024 entries) within the device's LDS (160 KiB on
+//   gfx950), so each row of a load is 64 contiguous bytes or more; their groups are dealt to the XCDs so that
+//   neighbouring groups run on one XCD and share the rest of each 128-byte line in its L2.
 // - Where only one or two workgroups fit per CU, each block walks several groups and prefetches the next one
 //   into registers while it transforms the current one.
 // - The twiddle table exp(-2 pi i j/n) is computed once per length in long double, rounded to FP64, and copied
@@ -43,7 +43,7 @@ constexpr int kFftLds = 2048;  // longest line
 constexpr int kContigEntries = GLASMA_FFT_CONTIG_ENTRIES;
 constexpr int kFftThreads = 256;
 constexpr int kMaxLinesPerBlock = 64;
-// strided lines per block at most.  8 would make each row of a load one 128-byte cache line, but fewer leave
+// strided lines per block at most for long lines.  8 would make each row of a load one 128-byte cache line, but fewer leave
 // room for more workgroups per CU: at 256^2 x 1024 with 8 components the y pass (length 256) takes 7.6 ms with
 // 8 lines (66 KiB of LDS, two workgroups per CU), 5.4 ms with 4 and 5.7 ms with 2; the z pass (length 1024)
 // 14.3 ms with 4 and 16.6 ms with 2.
@@ -51,6 +51,15 @@ constexpr int kMaxLinesPerBlock = 64;
 #define GLASMA_FFT_STRIDED_LINES 4
 #endif
 constexpr int kStridedLines = GLASMA_FFT_STRIDED_LINES;
+// shorter strided lines go more to a group, up to this many entries: a group of 256 entries gives its 256 threads one
+// element each, and its LDS stages, one radix-4 butterfly to four threads, are all latency.  Four packed arrays, plain
+// pass of length 128 at 128 x 128 x 256: 150 us with 512 entries, 125 with 1024, 143 with 2048, 198 with 4096;
+// filtered pass of length 64 at 128 x 128 x 64: 290 us with 128 entries (2 lines), 92 with 512, 74 with 1024, 71 with
+// 2048, 97 with 4096.
+#ifndef GLASMA_FFT_STRIDED_ENTRIES
+#define GLASMA_FFT_STRIDED_ENTRIES 1024
+#endif
+constexpr int kStridedEntries = GLASMA_FFT_STRIDED_ENTRIES;
 // the filtered z pass of fft_3d_poisson: lines per group.  With its two transforms per group the pass gains more
 // from a second workgroup per CU than from 64-byte rows: at 256^2 x 1024 (four arrays) 2 lines with twiddles from
 // memory (74 KiB of LDS) took 6.9-7.1 ms, 4 lines with the full twiddle table in LDS (155 KiB) 8.2 ms, 4 lines with
@@ -1003,7 +1012,8 @@ int fft_lines_filtered(hipStream_t st, double* data, int n, long es, long nlines
         while (2 * lpb * (n + 1) <= kContigEntries && 2 * lpb <= kMaxLinesPerBlock) lpb *= 2;
     } else {
         const size_t cap = dev.lds / (2 * sizeof(dbl2));  // entries per buffer
-        const int most = filt.on ? kFilterLines : kStridedLines;
+        int most = filt.on ? kFilterLines : kStridedLines;
+        while (2 * most * n <= kStridedEntries && 2 * most <= kMaxLinesPerBlock) most *= 2;
         while ((size_t)(2 * lpb) * (n + 1) <= cap && 2 * lpb <= most && 2 * lpb * n <= 16 * kFftThreads)
             lpb *= 2;
     }
