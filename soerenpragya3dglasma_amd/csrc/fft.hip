@@ -6,8 +6,8 @@
 //
 // Design: every transform is a set of independent 1D lines, transformed in groups.  A workgroup loads a group
 // into LDS (contiguous lines as one packed run; strided lines across the group, so neighbouring threads read
-// neighbouring addresses), runs a self-sorting Stockham transform in LDS (radix 4, 2, 3 kernels, any other
-// prime <= 13 by a direct DFT) and writes the lines back in place.  Multi-dimensional transforms are one pass per
+// neighbouring addresses), runs a self-sorting Stockham transform in LDS (radix 4, 2, 3, 5, 7, 11 and 13
+// butterflies in registers) and writes the lines back in place.  Multi-dimensional transforms are one pass per
 // axis, so each pass reads and writes the array once.
 // - Strided lines (the y and z passes) go 4 or more to a group (about 1024 entries) within the device's LDS (160 KiB on
 //   gfx950), so each row of a load is 64 contiguous bytes or more; their groups are dealt to the XCDs so that
@@ -108,7 +108,7 @@ __device__ __forceinline__ int nperm(int j, int n) { return (j & 1) ? n - ((j + 
 // Each block walks several groups and fetches the next group into registers (MAXE elements per thread) while
 // it transforms and stores the current one, so a CU keeps loads in flight through the LDS stages.  No block
 // waits for another.  TwLds: the twiddle table is copied into LDS once per block.
-template <bool TwLds, int MAXE, bool Filt>
+template <bool TwLds, int MAXE, bool Filt, int ODD>
 __global__ __launch_bounds__(kFftThreads) void k_fft_lines(double* __restrict__ data, Radices R, long es, long nlines,
                                                             long b1, long s1, long s2, int sign, int lpb, int ld,
                                                             long groups, long xcd_per, LineFilter filt,
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kFftThreads) void k_fft_lines(double* __restrict__ 
         const long gn = g + gstep;
         const bool more = gn < gend;
         if (more) fetch(gn);  // in flight during the stages and the stores below
-        int cur = stockham<Filt>(lds, bs, 0, R, lpb, ld, sign, tw);
+        int cur = stockham<Filt, ODD>(lds, bs, 0, R, lpb, ld, sign, tw);
         if (Filt) {  // strided lines only: this thread's line is myli, its positions idx >> lg_lpb
             dbl2* const fb = lds + cur * bs;
             const long t = (g * lpb + myli) % filt.P;
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kFftThreads) void k_fft_lines(double* __restrict__ 
                 }
             }
             __syncthreads();
-            cur = stockham<Filt>(lds, bs, cur, R, lpb, ld, -sign, tw);
+            cur = stockham<Filt, ODD>(lds, bs, cur, R, lpb, ld, -sign, tw);
         }
         const dbl2* const res = lds + cur * bs;
         const long base = start(g), lim = valid(g);
@@ -384,12 +384,16 @@ std::map<int, FftDevice> g_fft_dev;
 
 template <bool TW, int MAXE>
 hipError_t allow_lds(int v) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, false>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, v);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, v);
-    return e;
+    for (const void* f : {reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, false, 0>),
+                          reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, false, 1>),
+                          reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, false, 2>),
+                          reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, true, 0>),
+                          reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, true, 1>),
+                          reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, true, 2>)}) {
+        const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, v);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t fft_device(FftDevice* out) {
@@ -431,19 +435,19 @@ hipError_t fft_device(FftDevice* out) {
 #ifndef GLASMA_FFT_WALK_PER_CU
 #define GLASMA_FFT_WALK_PER_CU 2
 #endif
-template <bool TW, int MAXE, bool F>
+template <bool TW, int MAXE, bool F, int ODD>
 hipError_t launch_lines(hipStream_t st, size_t lds, int cus, double* data, const Radices& R, long es, long nlines,
                         long b1, long s1, long s2, int sign, int lpb, int ld, long groups, long xcd_per,
                         const LineFilter& filt, const dbl2* tw) {
     int per_cu = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, F>), kFftThreads, lds);
+        &per_cu, reinterpret_cast<const void*>(&k_fft_lines<TW, MAXE, F, ODD>), kFftThreads, lds);
     if (e != hipSuccess) return e;
     if (per_cu < 1) per_cu = 1;
     const long resident = per_cu <= GLASMA_FFT_WALK_PER_CU ? (long)cus * per_cu : groups;
     const long blocks = xcd_per > 0 ? 8 * std::min(xcd_per, (resident + 7) / 8) : std::min(groups, resident);
     if (blocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_fft_lines<TW, MAXE, F>), dim3((unsigned)blocks), dim3(kFftThreads), lds, st, data, R, es,
+    hipLaunchKernelGGL((k_fft_lines<TW, MAXE, F, ODD>), dim3((unsigned)blocks), dim3(kFftThreads), lds, st, data, R, es,
                        nlines, b1, s1, s2, sign, lpb, ld, groups, xcd_per, filt, tw);
     return hipGetLastError();
 }
@@ -1028,10 +1032,15 @@ int fft_lines_filtered(hipStream_t st, double* data, int n, long es, long nlines
     const size_t lds = bytes + (twlds ? sizeof(dbl2) * n : 0);
     const int need = (lpb * n + kFftThreads - 1) / kFftThreads;  // elements per thread
     const int maxe = need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : 16;
+    const int odd = odd_level(R);
     hipError_t ke;
-#define GLASMA_FFT_LAUNCH(TW, M, F)                                                                                 \
-    ke = launch_lines<TW, M, F>(st, lds, dev.cus, data, R, es, nlines, b1, s1, s2, sign, lpb, ld, groups, xcd_per, \
-                                filt, tw)
+#define GLASMA_FFT_LAUNCH_O(TW, M, F, O)                                                                              \
+    ke = launch_lines<TW, M, F, O>(st, lds, dev.cus, data, R, es, nlines, b1, s1, s2, sign, lpb, ld, groups, xcd_per, \
+                                   filt, tw)
+#define GLASMA_FFT_LAUNCH(TW, M, F)                      \
+    if (odd == 0) GLASMA_FFT_LAUNCH_O(TW, M, F, 0);      \
+    else if (odd == 1) GLASMA_FFT_LAUNCH_O(TW, M, F, 1); \
+    else GLASMA_FFT_LAUNCH_O(TW, M, F, 2)
 #define GLASMA_FFT_LAUNCH_M(TW, F)                   \
     switch (maxe) {                                  \
         case 2: GLASMA_FFT_LAUNCH(TW, 2, F); break;  \
@@ -1046,6 +1055,7 @@ int fft_lines_filtered(hipStream_t st, double* data, int n, long es, long nlines
     }
 #undef GLASMA_FFT_LAUNCH_M
 #undef GLASMA_FFT_LAUNCH
+#undef GLASMA_FFT_LAUNCH_O
     if (ke != hipSuccess)
         return fft_fail_hip(ke, "k_fft_lines launch (length " + std::to_string(n) + ", " + std::to_string(lpb) +
                                     " lines per block, " + std::to_string(lds) + " bytes of LDS)");

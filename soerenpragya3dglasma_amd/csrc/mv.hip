@@ -274,15 +274,15 @@ __global__ void __launch_bounds__(kPlaneThreads) k_sheet_plane(const double* __r
         lds[y * ld + i - y * g.nx] = dbl2{src[8 * i], src[8 * i + 1]};
     }
     __syncthreads();
-    int cur = stockham(lds, bs, 0, Rx, g.ny, ld, -1, tx);
-    cur = stockham(lds, bs, cur, Ry, g.nx, 1, -1, ty, ld);
+    int cur = stockham<false, 2>(lds, bs, 0, Rx, g.ny, ld, -1, tx);
+    cur = stockham<false, 2>(lds, bs, cur, Ry, g.nx, 1, -1, ty, ld);
     for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
         const int y = qdiv(i, g.nx, rnx), x = i - y * g.nx;
         lds[cur * bs + y * ld + x] *= sheet_filter(g, x, y, ax, ay, lam, meff);
     }
     __syncthreads();
-    cur = stockham(lds, bs, cur, Ry, g.nx, 1, +1, ty, ld);
-    cur = stockham(lds, bs, cur, Rx, g.ny, ld, +1, tx);
+    cur = stockham<false, 2>(lds, bs, cur, Ry, g.nx, 1, +1, ty, ld);
+    cur = stockham<false, 2>(lds, bs, cur, Rx, g.ny, ld, +1, tx);
     for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
         const int y = qdiv(i, g.nx, rnx);
         A[(long)blockIdx.x * g.P + i] = lds[cur * bs + y * ld + i - y * g.nx];
@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom
             lds[li * ld + z] = v;
         }
         __syncthreads();
-        int cur = stockham<true>(lds, bs, 0, R, lpb, ld, -1, tw);
+        int cur = stockham<true, 2>(lds, bs, 0, R, lpb, ld, -1, tw);
         for (int i = threadIdx.x; i < lpb * n; i += 256) {
             const int li = i & (lpb - 1), k = i >> lg;
             dbl2 f = h[2 * k <= n ? k : n - k];
@@ -572,7 +572,7 @@ __global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom
             *at = cmul(f, *at);
         }
         __syncthreads();
-        cur = stockham<true>(lds, bs, cur, R, lpb, ld, +1, tw);
+        cur = stockham<true, 2>(lds, bs, cur, R, lpb, ld, +1, tw);
         for (int i = threadIdx.x; i < lpb * n; i += 256) {
             const int li = i & (lpb - 1), z = i >> lg;
             const long s2 = s0 + li;
