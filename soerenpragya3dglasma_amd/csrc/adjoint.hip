@@ -194,11 +194,14 @@ int run_segment(glasma_ctx* ctx, const std::vector<State>& seg, const std::vecto
     return 0;
 }
 
-// the gradient's second stream and its events (default priority, kept in the context)
-int ensure_seg_stream(glasma_ctx* ctx) {
+// the gradient's second stream and its events, one per set and one more (default priority, kept in the context)
+int ensure_seg_stream(glasma_ctx* ctx, int nset) {
     if (!ctx->stream2) GL_HIP(ctx, hipStreamCreate(&ctx->stream2));
-    for (hipEvent_t& ev : ctx->seg_ev)
-        if (!ev) GL_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    while ((int)ctx->seg_ev.size() <= nset) {
+        hipEvent_t ev = nullptr;
+        GL_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        ctx->seg_ev.push_back(ev);
+    }
     return 0;
 }
 
@@ -346,70 +349,98 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
     const int nseg = (nsteps + ckpt - 1) / ckpt;
     const int seglen = nsteps < ckpt ? nsteps : ckpt;
     int rc = 0;
-    DevBuf b;
-    IcTape tape;
-    double* rho_d = b.get(ctx, 8 * S, &rc);
-    tape.rho_s = rc ? nullptr : b.get(ctx, 8 * S, &rc);
-    tape.A0 = rc ? nullptr : b.get(ctx, 8 * S, &rc);
-    tape.A1 = rc ? nullptr : b.get(ctx, 8 * S, &rc);
-    tape.V0 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
-    tape.V1 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
-    // checkpoints at the starts of all segments but the last, whose states the forward run leaves in the segment
-    // slots; the slots in two sets (segment sg uses set sg % 2), so that one segment's recompute, on the second
-    // stream, overlaps the backward sweep of the segment after it, when the second set takes at most a quarter of the
-    // device memory (else one set, each segment recomputed just before its sweep)
-    int nset = 1;
+    // The segment slots are kept in nset sets (segment sg uses set sg % nset).  The forward run leaves the states of the
+    // last nset segments in them; an earlier segment starts from a checkpoint and is recomputed into its set, on the
+    // second stream, once the sweep over the segment that held the set is done, beside the sweeps of the segments in
+    // between.  As many sets as a quarter of the device memory holds (two where one takes no more than that quarter,
+    // one beyond): a recomputed step costs a forward step, so the gradient of 100 steps with checkpoints every 20 at
+    // 48 x 48 x 128 took 78 ms with four of five segments recomputed, 77, 73 and 70 with two, three and four
+    // kept and 67 with all five (38 GB).
+    int nset = 1, nset0 = 1;  // nset0: without the sets beyond two
     if (nseg > 1) {
-        size_t freeb = 0, totalb = 0;
+        size_t freeb = 0, totalb = 0, held = 0;
+        for (const auto& p : ctx->wpool) held += p.first * sizeof(double);
         const size_t set_bytes = (size_t)seglen * (2 * kUPlanes + kEPlanes + kJPlanes) * Sp * sizeof(double);
-        if (hipMemGetInfo(&freeb, &totalb) == hipSuccess && set_bytes <= totalb / 4) nset = 2;
-        const char* env = std::getenv("GLASMA_GRAD_SETS");  // 1: one set always (read on every call)
-        if (env && std::atoi(env) == 1) nset = 1;
-    }
-    // ck[0] is the initial state in the context's fields, which no step writes; tmp: the forward run's other states
-    std::vector<State> ck(nseg > 1 ? nseg - 1 : 0), seg[2], tmp(nseg > 1 ? 2 : 0);
-    std::vector<double*> Uh[2];
-    for (size_t k = 1; k < ck.size(); k++) {
-        ck[k].U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
-        ck[k].E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
-        ck[k].J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
-    }
-    for (auto& s : tmp) {
-        s.U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
-        s.E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
-        s.J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
-    }
-    for (int q = 0; q < nset; q++) {
-        seg[q].resize(seglen + 1);
-        for (size_t i = 1; i < seg[q].size(); i++) {  // seg[q][0] is the segment's first state itself
-            seg[q][i].U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
-            seg[q][i].E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
-            seg[q][i].J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+        if (hipMemGetInfo(&freeb, &totalb) == hipSuccess) {
+            if (set_bytes <= totalb / 4) nset = 2;
+            nset0 = nset;
+            while (nset < nseg && (size_t)(nset + 1) * set_bytes <= std::min(totalb / 4, (freeb + held) / 2)) nset++;
         }
-        Uh[q].resize(seglen > 0 ? seglen : 0);
-        for (auto& p : Uh[q]) p = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+        const char* env = std::getenv("GLASMA_GRAD_SETS");  // that many sets at most (read on every call)
+        if (env && std::atoi(env) >= 1) nset = std::min(nset, std::atoi(env));
+        nset0 = std::min(nset0, nset);
     }
-    double* cU[2];
-    double* cJ[2];
-    cU[0] = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
-    cU[1] = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
-    cJ[0] = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
-    cJ[1] = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
-    double* cE = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
-    double* rho_bar = rc ? nullptr : b.get(ctx, 8 * S, &rc);
-    double* work = rc ? nullptr : b.get(ctx, 54 * Sp + 36 * Sp + 32 * S, &rc);
+    int nrec = 0;  // segments to recompute: the first nrec
+    IcTape tape;
+    double *rho_d, *cU[2], *cJ[2], *cE, *rho_bar, *work;
+    // ck[0] is the initial state in the context's fields, which no step writes; tmp: the forward run's other states
+    std::vector<State> ck, tmp;
+    std::vector<std::vector<State>> seg;
+    std::vector<std::vector<double*>> Uh;
+    auto allocate = [&]() {
+        DevBuf b;
+        nrec = nseg > nset ? nseg - nset : 0;
+        ck.assign(nrec, State());
+        tmp.assign(nrec > 0 ? 2 : 0, State());
+        seg.assign(nset, {});
+        Uh.assign(nset, {});
+        rho_d = b.get(ctx, 8 * S, &rc);
+        tape.rho_s = rc ? nullptr : b.get(ctx, 8 * S, &rc);
+        tape.A0 = rc ? nullptr : b.get(ctx, 8 * S, &rc);
+        tape.A1 = rc ? nullptr : b.get(ctx, 8 * S, &rc);
+        tape.V0 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
+        tape.V1 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
+        for (size_t k = 1; k < ck.size(); k++) {
+            ck[k].U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+            ck[k].E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
+            ck[k].J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+        }
+        for (auto& s : tmp) {
+            s.U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+            s.E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
+            s.J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+        }
+        for (int q = 0; q < nset; q++) {
+            seg[q].resize(seglen + 1);
+            for (size_t i = 1; i < seg[q].size(); i++) {  // seg[q][0] is the segment's first state itself
+                seg[q][i].U = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+                seg[q][i].E = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
+                seg[q][i].J = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+            }
+            Uh[q].resize(seglen > 0 ? seglen : 0);
+            for (auto& p : Uh[q]) p = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+        }
+        cU[0] = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+        cU[1] = rc ? nullptr : b.get(ctx, kUPlanes * Sp, &rc);
+        cJ[0] = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+        cJ[1] = rc ? nullptr : b.get(ctx, kJPlanes * Sp, &rc);
+        cE = rc ? nullptr : b.get(ctx, kEPlanes * Sp, &rc);
+        rho_bar = rc ? nullptr : b.get(ctx, 8 * S, &rc);
+        work = rc ? nullptr : b.get(ctx, 54 * Sp + 36 * Sp + 32 * S, &rc);
+    };
+    allocate();
+    if (rc && nset > nset0) {  // another user took the memory meanwhile: without the extra sets
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(ctx->stream);
+        for (auto& p : ctx->wpool) (void)hipFree(p.second);
+        ctx->wpool.clear();
+        nset = nset0;
+        rc = 0;
+        allocate();
+    }
     if (rc) return rc;
-    if (nset > 1 && (rc = ensure_seg_stream(ctx))) return rc;
+    const bool second = nset > 1 && nrec > 0;  // recomputes go on the second stream
+    if (second && (rc = ensure_seg_stream(ctx, nset))) return rc;
     std::vector<double> h;
     rho_to_dev_layout(ctx, rho, h);
     GL_HIP(ctx, hipMemcpy(rho_d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
-    // forward, every step out of place: the segments before the last from the initial state in the context's fields
+    // forward, every step out of place: the segments to recompute from the initial state in the context's fields
     // (left as they are), each checkpoint written by the step that reaches it and the other states alternating between
-    // the two tmp states; then the last segment into the segment slots, so that its backward sweep recomputes nothing
+    // the two tmp states; then the rest into the segment slots, whose sweeps need no recompute
     if ((rc = ic_left_from_charge(ctx, mv, rho_d, tape))) return rc;
-    const int nlast = nseg > 0 ? (nseg - 1) * ckpt : 0;
+    const int nlast = nrec * ckpt;
     State fin = {ctx->U[ctx->cur], ctx->E, ctx->J[ctx->cur]};
-    if (nseg > 1) ck[0] = fin;
+    if (nrec > 0) ck[0] = fin;
     for (int n = 0; n < nlast; n++) {
         const State nx = ((n + 1) % ckpt == 0 && n + 1 < nlast) ? ck[(n + 1) / ckpt] : tmp[n & 1];
         StepArgs F = step_args(ctx, ctx->cur, false);
@@ -422,11 +453,11 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
         if ((rc = launch_step_args(ctx, F))) return rc;
         fin = nx;
     }
-    if (nseg > 0) {
-        const int q = (nseg - 1) % nset;
+    for (int sg = nrec; sg < nseg; sg++) {
+        const int q = sg % nset, len = std::min(ckpt, nsteps - sg * ckpt);
         seg[q][0] = fin;
-        if ((rc = run_segment(ctx, seg[q], Uh[q], nsteps - nlast))) return rc;
-        fin = seg[q][nsteps - nlast];
+        if ((rc = run_segment(ctx, seg[q], Uh[q], len))) return rc;
+        fin = seg[q][len];
     }
     GL_HIP(ctx, hipGetLastError());
     if ((rc = slab_energy(ctx, zc, half, energy, fin.U, fin.E))) return rc;
@@ -440,31 +471,13 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
         A.Eb = cE;
         hipLaunchKernelGGL(k_slab_vjp, agrid(S), dim3(kAdjBlock), 0, ctx->stream, A, cU[0]);
     }
-    // events: seg_ev[q] the recompute into set q done (second stream), seg_ev[2 + q] the sweep over set q done (the
-    // context's stream), seg_ev[4] the forward run done (the checkpoints written)
-    hipEvent_t* ev = ctx->seg_ev;
-    if (nset > 1) {
-        GL_HIP(ctx, hipEventRecord(ev[4], ctx->stream));
-        GL_HIP(ctx, hipStreamWaitEvent(ctx->stream2, ev[4], 0));
-    }
+    // events: seg_ev[q] the recompute into set q done (second stream), seg_ev[nset] the latest sweep done (the context's
+    // stream; each wait follows its record, and the checkpoints are written before the first)
     int cb = 0;
-    // backward sweep, one segment at a time; with two sets the recompute of segment sg - 1 is queued on the second
-    // stream first
     for (int sg = nseg - 1; sg >= 0; sg--) {
         const int n0 = sg * ckpt, n1 = (n0 + ckpt < nsteps) ? n0 + ckpt : nsteps;
         const int q = sg % nset;
-        if (nset == 1 && sg < nseg - 1) {
-            seg[0][0] = ck[sg];
-            if ((rc = run_segment(ctx, seg[0], Uh[0], ckpt))) return rc;
-        }
-        if (nset > 1 && sg >= 1) {
-            const int q1 = (sg - 1) & 1;  // the set the sweep of segment sg + 1 read
-            if (sg + 1 <= nseg - 1) GL_HIP(ctx, hipStreamWaitEvent(ctx->stream2, ev[2 + q1], 0));
-            seg[q1][0] = ck[sg - 1];
-            if ((rc = run_segment(ctx, seg[q1], Uh[q1], ckpt, ctx->stream2))) return rc;
-            GL_HIP(ctx, hipEventRecord(ev[q1], ctx->stream2));
-        }
-        if (nset > 1 && sg < nseg - 1) GL_HIP(ctx, hipStreamWaitEvent(ctx->stream, ev[q], 0));
+        if (second && sg < nrec) GL_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->seg_ev[q], 0));
         for (int n = n1 - 1; n >= n0; n--) {
             const int i = n - n0;
             StepAdjArgs A = adj_args(ctx);
@@ -481,7 +494,15 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
             if ((rc = run_vjp(ctx, A))) return rc;
             cb ^= 1;
         }
-        if (nset > 1 && sg >= 2) GL_HIP(ctx, hipEventRecord(ev[2 + q], ctx->stream));  // set q: next for sg - 2
+        if (sg >= nset) {  // the set is free: segment sg - nset into it
+            if (second) {
+                GL_HIP(ctx, hipEventRecord(ctx->seg_ev[nset], ctx->stream));
+                GL_HIP(ctx, hipStreamWaitEvent(ctx->stream2, ctx->seg_ev[nset], 0));
+            }
+            seg[q][0] = ck[sg - nset];
+            if ((rc = run_segment(ctx, seg[q], Uh[q], ckpt, second ? ctx->stream2 : ctx->stream))) return rc;
+            if (second) GL_HIP(ctx, hipEventRecord(ctx->seg_ev[q], ctx->stream2));
+        }
     }
     // the context's fields and UOld still hold the initial state (the linearisation point of the initial-condition
     // map): no step above wrote them

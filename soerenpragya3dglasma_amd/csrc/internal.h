@@ -69,7 +69,7 @@ struct glasma_ctx {
     // second stream and events of the gradient call (created on first use, default priority): a checkpoint segment's
     // recompute there overlaps the previous segment's backward sweep
     hipStream_t stream2 = nullptr;
-    hipEvent_t seg_ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    std::vector<hipEvent_t> seg_ev;
     std::string err;
 };
 
