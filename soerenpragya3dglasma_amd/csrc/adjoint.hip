@@ -1,8 +1,8 @@
 // Reverse-mode derivatives on the device (no counterpart in the reference, which has no gradient code):
 // the leapfrog step (two passes per step, no atomics: A with B folded in, then the staple gather), the slab
 // energy, and the whole map charge density -> left-moving MV sheet -> nsteps leapfrog steps -> slab energy, with
-// the forward run checkpointed every ckpt steps and each segment but the last recomputed once during the backward
-// sweep.
+// the forward run checkpointed every ckpt steps: the last segments, as many as the memory holds, are kept whole, each
+// earlier one is recomputed once during the backward sweep.
 #include <cstdlib>
 #include <cstring>
 #include <vector>

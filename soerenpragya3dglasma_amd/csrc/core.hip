@@ -716,6 +716,8 @@ int glasma_destroy(glasma_ctx* ctx) {
         if (w.second) (void)hipFree(w.second);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
+    if (ctx->monitors) hipHostFree(ctx->monitors);
+    if (ctx->monitors_ev) hipEventDestroy(ctx->monitors_ev);
     for (hipEvent_t ev : ctx->seg_ev)
         if (ev) hipEventDestroy(ev);
     if (ctx->stream) hipStreamDestroy(ctx->stream);

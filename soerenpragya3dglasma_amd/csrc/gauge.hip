@@ -622,33 +622,56 @@ __global__ __launch_bounds__(kCgBlock) void k_cg_update(const double* __restrict
     block_partials(ssq, 0.0, sm, 0.0, part + 4 * (long)blockIdx.x);
 }
 
-// fixed-order reduction of block partials: block i takes partials [i per, (i + 1) per), strided per-thread sums then the
-// block tree, into out + 4 i
-__global__ __launch_bounds__(kCgBlock) void k_cg_reduce(const double* __restrict__ part, long nblk, long per,
-                                                         double* __restrict__ out, double fm0) {
-    double s0 = 0, s1 = 0, m0 = 0, m1 = fm0;
-    const long end = min(nblk, (long)(blockIdx.x + 1) * per);
-    for (long b = (long)blockIdx.x * per + threadIdx.x; b < end; b += blockDim.x) {
+// fixed-order reduction of block partials: block (i, y) takes partials [i per, (i + 1) per) of set y, strided per-thread
+// sums then the block tree, into out + 4 i of that set
+struct CgPartials {
+    const double* part[2];
+    long n[2], per[2];
+    double fm0[2];
+    double* out[2];
+};
+__global__ __launch_bounds__(kCgBlock) void k_cg_reduce(CgPartials r) {
+    const int y = blockIdx.y;
+    const double* const part = r.part[y];
+    double s0 = 0, s1 = 0, m0 = 0, m1 = r.fm0[y];
+    const long end = min(r.n[y], (long)(blockIdx.x + 1) * r.per[y]);
+    for (long b = (long)blockIdx.x * r.per[y] + threadIdx.x; b < end; b += blockDim.x) {
         s0 += part[4 * b];
         s1 += part[4 * b + 1];
         m0 = fmax(m0, part[4 * b + 2]);
         m1 = fmin(m1, part[4 * b + 3]);
     }
-    block_partials(s0, s1, m0, m1, out + 4 * (long)blockIdx.x);
+    block_partials(s0, s1, m0, m1, r.out[y] + 4 * (long)blockIdx.x);
 }
 
-// the four monitors of nblk block partials into out[0..3]: one block up to 4096 partials, else up to 256 blocks of
-// 1024 or more into tmp (4 * 256 doubles) and one block over those (a single block over 262144 partials took 0.25 ms)
+// the four monitors of nset sets of block partials, into out + 4 k for set k: one block a set up to 4096 partials, else
+// up to 256 blocks of 1024 or more into tmp (4 * 256 doubles a set) and one block over those (a single block over 262144
+// partials took 0.25 ms)
 constexpr long kReduceTmp = 4 * 256;
-void reduce_partials(hipStream_t st, const double* part, long nblk, double* out, double fm0, double* tmp) {
-    if (nblk <= 4096) {
-        hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(kCgBlock), 0, st, part, nblk, nblk, out, fm0);
-        return;
+void reduce_partials(hipStream_t st, int nset, const double* const* part, const long* n, const double* fm0, double* out,
+                     double* tmp) {
+    CgPartials r;
+    long most = 0;
+    for (int k = 0; k < nset; k++) most = std::max(most, n[k]);
+    const long nb2 = most <= 4096 ? 1 : std::min(256L, (most + 1023) / 1024);
+    for (int k = 0; k < nset; k++) {
+        r.part[k] = part[k];
+        r.n[k] = n[k];
+        r.per[k] = (n[k] + nb2 - 1) / nb2;
+        r.fm0[k] = fm0[k];
+        r.out[k] = nb2 == 1 ? out + 4 * k : tmp + kReduceTmp * k;
     }
-    const long nb2 = std::min(256L, (nblk + 1023) / 1024);
-    const long per = (nblk + nb2 - 1) / nb2;
-    hipLaunchKernelGGL(k_cg_reduce, dim3((unsigned)nb2), dim3(kCgBlock), 0, st, part, nblk, per, tmp, fm0);
-    hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(kCgBlock), 0, st, tmp, nb2, nb2, out, fm0);
+    hipLaunchKernelGGL(k_cg_reduce, dim3((unsigned)nb2, nset), dim3(kCgBlock), 0, st, r);
+    if (nb2 == 1) return;
+    for (int k = 0; k < nset; k++) {
+        r.part[k] = r.out[k];
+        r.n[k] = r.per[k] = nb2;
+        r.out[k] = out + 4 * k;
+    }
+    hipLaunchKernelGGL(k_cg_reduce, dim3(1, nset), dim3(kCgBlock), 0, st, r);
+}
+void reduce_partials(hipStream_t st, const double* part, long nblk, double* out, double fm0, double* tmp) {
+    reduce_partials(st, 1, &part, &nblk, &fm0, out, tmp);
 }
 
 // ---- Gauss-law restoration (GAUSSLAWFIXING/GaussRestore.cpp, GaussRestore2D.cpp) -------------------------
@@ -735,6 +758,13 @@ int ensure_gauge(glasma_ctx* ctx) {
     return 0;
 }
 
+// host memory for the eight monitors of an iteration and the event that says they are there (kept in the context)
+int ensure_monitors(glasma_ctx* ctx) {
+    if (!ctx->monitors) GL_HIP(ctx, hipHostMalloc(&ctx->monitors, 8 * sizeof(double), hipHostMallocDefault));
+    if (!ctx->monitors_ev) GL_HIP(ctx, hipEventCreateWithFlags(&ctx->monitors_ev, hipEventDisableTiming));
+    return 0;
+}
+
 int ensure_gauge_fixed(glasma_ctx* ctx) {
     if (!ctx->UG) GL_HIP(ctx, hipMalloc(&ctx->UG, (size_t)kUPlanes * pad_sites(ctx->g.S) * sizeof(double)));
     if (!ctx->EG) GL_HIP(ctx, hipMalloc(&ctx->EG, (size_t)kEPlanes * pad_sites(ctx->g.S) * sizeof(double)));
@@ -785,7 +815,8 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
                     kCgBlock % g.nx == 0 && factorize(g.nx, R) == 0 && fft_twiddles(g.nx, &tw) == hipSuccess;
     (void)hipGetLastError();
     const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g, xf);
-    rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + kReduceTmp);
+    rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + 2 * kReduceTmp);
+    if (!rc) rc = ensure_monitors(ctx);
     if (!rc && algo != GLASMA_GAUGE_LOS_ALAMOS) rc = ensure_fftbuf(ctx, 8 * (size_t)g.S);  // 4 complex per site
     if (rc) return rc;
     const double* a = ctx->p.a;
@@ -794,9 +825,9 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     const double cx = (1.0 / a[0]) * (1.0 / a[0]), cy = (1.0 / a[1]) * (1.0 / a[1]), cz = (1.0 / a[2]) * (1.0 / a[2]);
     const double fm0 = 6.0 * (1.0 / (a[0] * a[0]) + 1.0 / (a[1] * a[1]) + 1.0 / (a[2] * a[2]));
     double* part = ctx->red;                // 2 * nblk blocks of 4 (Los Alamos: both half sweeps)
-    double* spart = ctx->red + 8 * nblk;    // Los Alamos step monitors
-    double* fin = ctx->red + 16 * nblk;
-    double* tmp = fin + 8;
+    double* spart = ctx->red + 8 * nblk;    // step monitors (Los Alamos: both half sweeps)
+    double* tmp = ctx->red + 16 * nblk + 8;
+    double* h = ctx->monitors;              // host memory: the reduction writes the eight monitors straight to it
     double* F = ctx->fftbuf;
     // Los Alamos sweeps read U^G; the Fourier and Jacobi iterations form it on the fly (k_cg_dev_fused) and keep
     // the reference's lag of the top ghost layer by synchronising Gtop right after each deviation kernel, where
@@ -806,8 +837,33 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     double gmax = 1.0, gavg = 0.0, smax = 0.0, savg = 0.0, fmin = 0.0, fsum = 0.0;
     int n = 0;
     const double V = (double)g.S;
+    // the deviation kernel of one Fourier or Jacobi iteration (reads G, writes F and part)
+    auto deviation = [&]() {
+#define GLASMA_CG_DEV(C, X)                                                                                     \
+    if (walk.zc)                                                                                                 \
+        hipLaunchKernelGGL((k_cg_dev_walk<C, X>), dim3(walk.n), dim3(kCgBlock), 0, ctx->stream,                     \
+                           ctx->U[ctx->cur], ctx->G, ctx->Gtop, F, part, g, cx, cy, cz, fm0, walk, R, tw);         \
+    else                                                                                                         \
+        hipLaunchKernelGGL((k_cg_dev_fused<C, X>), dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream,           \
+                           ctx->U[ctx->cur], ctx->G, ctx->Gtop, F, part, g, cx, cy, cz, fm0, ord, R, tw)
+        if (cons) {
+            if (xf) {
+                GLASMA_CG_DEV(true, true);
+            } else {
+                GLASMA_CG_DEV(true, false);
+            }
+        } else {
+            if (xf) {
+                GLASMA_CG_DEV(false, true);
+            } else {
+                GLASMA_CG_DEV(false, false);
+            }
+            hipLaunchKernelGGL(k_cg_sync_top, grid1(g.P), dim3(kCgBlock), 0, ctx->stream, ctx->G, ctx->Gtop, g);
+        }
+#undef GLASMA_CG_DEV
+    };
+    bool queued = false;  // the next iteration's deviation kernel is already in the stream
     while (n < maxit && gmax > tol) {
-        double h[8];
         if (algo == GLASMA_GAUGE_LOS_ALAMOS) {
             for (int parity = 0; parity < 2; parity++) {
                 hipLaunchKernelGGL(k_cg_losalamos, dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream, ctx->UG, ctx->G,
@@ -815,32 +871,8 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
                                    ord);
                 if ((rc = transform_links(ctx))) return rc;
             }
-            reduce_partials(ctx->stream, part, 2 * nblk, fin, fm0, tmp);
-            reduce_partials(ctx->stream, spart, 2 * nblk, fin + 4, 0.0, tmp);
         } else {
-#define GLASMA_CG_DEV(C, X)                                                                                     \
-    if (walk.zc)                                                                                                 \
-        hipLaunchKernelGGL((k_cg_dev_walk<C, X>), dim3(walk.n), dim3(kCgBlock), 0, ctx->stream,            \
-                           ctx->U[ctx->cur], ctx->G, ctx->Gtop, F, part, g, cx, cy, cz, fm0, walk, R, tw);         \
-    else                                                                                                         \
-        hipLaunchKernelGGL((k_cg_dev_fused<C, X>), dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream,           \
-                           ctx->U[ctx->cur], ctx->G, ctx->Gtop, F, part, g, cx, cy, cz, fm0, ord, R, tw)
-            if (cons) {
-                if (xf) {
-                    GLASMA_CG_DEV(true, true);
-                } else {
-                    GLASMA_CG_DEV(true, false);
-                }
-            } else {
-                if (xf) {
-                    GLASMA_CG_DEV(false, true);
-                } else {
-                    GLASMA_CG_DEV(false, false);
-                }
-                hipLaunchKernelGGL(k_cg_sync_top, grid1(g.P), dim3(kCgBlock), 0, ctx->stream, ctx->G, ctx->Gtop, g);
-            }
-#undef GLASMA_CG_DEV
-            reduce_partials(ctx->stream, part, walk.zc ? (long)walk.n : nblk, fin, fm0, tmp);
+            if (!queued) deviation();
             if (cons) {
                 // the Laplacian of the links that exist (open z: the Neumann Laplacian, a cosine transform in z); the
                 // zero mode (zero by construction) dropped
@@ -871,15 +903,24 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
             }
             if (xf)
                 hipLaunchKernelGGL(k_cg_update<true>, dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream, F, ctx->G,
-                                   part, g, param, R, tw);
+                                   spart, g, param, R, tw);
             else
                 hipLaunchKernelGGL(k_cg_update<false>, dim3((unsigned)nblk), dim3(kCgBlock), 0, ctx->stream, F, ctx->G,
-                                   part, g, param, R, tw);
-            reduce_partials(ctx->stream, part, nblk, fin + 4, 0.0, tmp);
-            GL_HIP(ctx, hipGetLastError());
+                                   spart, g, param, R, tw);
         }
-        GL_HIP(ctx, hipMemcpyAsync(h, fin, 8 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        const double* const sets[2] = {part, spart};
+        const long counts[2] = {!fused ? 2 * nblk : walk.zc ? (long)walk.n : nblk, fused ? nblk : 2 * nblk};
+        const double mins[2] = {fm0, 0.0};
+        reduce_partials(ctx->stream, 2, sets, counts, mins, h, tmp);
+        GL_HIP(ctx, hipGetLastError());
+        GL_HIP(ctx, hipEventRecord(ctx->monitors_ev, ctx->stream));
+        // On small lattices the next iteration's deviation kernel runs while the host reads this one's monitors: it
+        // changes nothing that the end of the call uses (not G; Gtop as the end of the call sets it).  That saves 7.5 us
+        // an iteration and costs one deviation kernel where the tolerance ends the call: 21 us at 32 x 40 x 64, 85 at
+        // 64 x 64 x 128, hence the limit of 512 blocks (131072 sites, about 30 us).
+        queued = fused && n + 1 < maxit && nblk <= 512;
+        if (queued) deviation();
+        GL_HIP(ctx, hipEventSynchronize(ctx->monitors_ev));
         gmax = h[2];
         gavg = std::sqrt(h[0] / (V * 8.0));
         fmin = h[3];

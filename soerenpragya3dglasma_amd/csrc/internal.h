@@ -70,6 +70,9 @@ struct glasma_ctx {
     // recompute there overlaps the previous segment's backward sweep
     hipStream_t stream2 = nullptr;
     std::vector<hipEvent_t> seg_ev;
+    // gauge fixing: the monitors of an iteration in host memory, and the event after their reduction
+    double* monitors = nullptr;
+    hipEvent_t monitors_ev = nullptr;
     std::string err;
 };
 
