@@ -34,6 +34,12 @@ int ensure_red(glasma_ctx* ctx, size_t doubles) {
     ctx->red_cap = doubles;
     return 0;
 }
+// the host memory for small results and its event (kept in the context)
+int ensure_host_out(glasma_ctx* ctx) {
+    if (!ctx->host_out) GL_HIP(ctx, hipHostMalloc(&ctx->host_out, kHostOut * sizeof(double), hipHostMallocDefault));
+    if (!ctx->host_ev) GL_HIP(ctx, hipEventCreateWithFlags(&ctx->host_ev, hipEventDisableTiming));
+    return 0;
+}
 int ensure_fftbuf(glasma_ctx* ctx, size_t doubles) {
     if (ctx->fftbuf_cap >= doubles) return 0;
     if (ctx->fftbuf) (void)hipFree(ctx->fftbuf);
@@ -516,19 +522,28 @@ __global__ void k_tmap_finalize(const double* __restrict__ part, double* __restr
 // wavefront per output: lane l adds the blocks l, l + 64, ... in order, then the lanes are added in a fixed tree, so
 // the result does not depend on scheduling.  One thread per output was a chain of bpp dependent adds on strided
 // loads: 107 us at 256 x 256 x 512 (bpp = 256).
-__global__ void __launch_bounds__(256) k_finalize(const double* __restrict__ red, double* __restrict__ out, int nz,
-                                                  int bpp, int K, unsigned maxmask) {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= nz * K) return;
-    const int z = i / K, k = i % K;
-    const bool mx = (maxmask >> k) & 1u;
-    double acc = 0.0;
-    for (int b = lane; b < bpp; b += 64) {
-        const double v = red[((long)z * bpp + b) * K + k];
-        acc = mx ? fmax(acc, v) : acc + v;
+//
+// A block takes 16 outputs and writes them together: `out` may be host memory, where a lone 8-byte store is a transfer
+// of its own.
+constexpr int kFinOuts = 16;
+__global__ void __launch_bounds__(64 * kFinOuts) k_finalize(const double* __restrict__ red, double* __restrict__ out,
+                                                            int nz, int bpp, int K, unsigned maxmask) {
+    __shared__ double sh[kFinOuts];
+    const int w = threadIdx.x >> 6, i = blockIdx.x * kFinOuts + w, lane = threadIdx.x & 63;
+    if (i < nz * K) {
+        const int z = i / K, k = i % K;
+        const bool mx = (maxmask >> k) & 1u;
+        double acc = 0.0;
+        for (int b = lane; b < bpp; b += 64) {
+            const double v = red[((long)z * bpp + b) * K + k];
+            acc = mx ? fmax(acc, v) : acc + v;
+        }
+        acc = mx ? wave_max(acc) : wave_sum(acc);
+        if (lane == 0) sh[w] = acc;
     }
-    acc = mx ? wave_max(acc) : wave_sum(acc);
-    if (lane == 0) out[i] = acc;
+    __syncthreads();
+    const int o = blockIdx.x * kFinOuts + threadIdx.x;
+    if (threadIdx.x < kFinOuts && o < nz * K) out[o] = sh[threadIdx.x];
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -614,6 +629,7 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     const Geom& g = ctx->g;
     const int bpp = (int)((g.P + 255) / 256);
     int rc = ensure_red(ctx, (size_t)g.nz * bpp * K + (size_t)g.nz * K);
+    if (!rc) rc = ensure_host_out(ctx);
     if (rc) return rc;
     ObsArgs A;
     A.U = ctx->U[ctx->cur];
@@ -627,12 +643,18 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
     hipLaunchKernelGGL(kern, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A);
     GL_HIP(ctx, hipGetLastError());
-    double* fin = ctx->red + (size_t)g.nz * bpp * K;
+    // results that fit go straight to pinned host memory: a copy to pageable memory is a launch, a staging copy and their
+    // gaps (six records of 64 x 56 x 96 took 528 us with the copies and 472 without)
     const int n = g.nz * K;
-    hipLaunchKernelGGL(k_finalize, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, ctx->red, fin, g.nz, bpp, K, maxmask);
+    const bool direct = n <= kHostOut;
+    double* fin = direct ? ctx->host_out : ctx->red + (size_t)g.nz * bpp * K;
+    hipLaunchKernelGGL(k_finalize, dim3((n + kFinOuts - 1) / kFinOuts), dim3(64 * kFinOuts), 0, ctx->stream, ctx->red, fin,
+                       g.nz, bpp, K, maxmask);
     per_z.resize(n);
-    GL_HIP(ctx, hipMemcpyAsync(per_z.data(), fin, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if (!direct)
+        GL_HIP(ctx, hipMemcpyAsync(per_z.data(), fin, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (direct) std::memcpy(per_z.data(), fin, n * sizeof(double));
     return 0;
 }
 
@@ -716,8 +738,8 @@ int glasma_destroy(glasma_ctx* ctx) {
         if (w.second) (void)hipFree(w.second);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
-    if (ctx->monitors) hipHostFree(ctx->monitors);
-    if (ctx->monitors_ev) hipEventDestroy(ctx->monitors_ev);
+    if (ctx->host_out) (void)hipHostFree(ctx->host_out);
+    if (ctx->host_ev) hipEventDestroy(ctx->host_ev);
     for (hipEvent_t ev : ctx->seg_ev)
         if (ev) hipEventDestroy(ev);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
@@ -879,7 +901,8 @@ int glasma_bulk_noalloc(glasma_ctx* ctx, double* out9) {
     double* fin = ptr + (long)g.nz * bpp * 9;
     double* tot = fin + (long)g.nz * 9;
     hipLaunchKernelGGL(k_bulk, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A);
-    hipLaunchKernelGGL(k_finalize, dim3((g.nz * 9 + 3) / 4), dim3(256), 0, ctx->stream, ptr, fin, g.nz, bpp, 9, 0u);
+    hipLaunchKernelGGL(k_finalize, dim3((g.nz * 9 + kFinOuts - 1) / kFinOuts), dim3(64 * kFinOuts), 0, ctx->stream, ptr, fin,
+                       g.nz, bpp, 9, 0u);
     hipLaunchKernelGGL(k_sum_layers, dim3(1), dim3(64), 0, ctx->stream, fin, tot, g.nz, 9);
     GL_HIP(ctx, hipGetLastError());
     GL_HIP(ctx, hipMemcpyAsync(out9, tot, 9 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -990,6 +1013,7 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     const int bpp = (int)((g.P + 255) / 256);
     const int chunk = map_chunk(g), nchunk = (g.nz + chunk - 1) / chunk;
     int rc = ensure_red(ctx, (size_t)(nchunk + 1) * 2 * g.P);
+    if (!rc) rc = ensure_host_out(ctx);
     if (rc) return rc;
     ObsArgs A;
     A.U = ctx->U[ctx->cur];
@@ -1001,12 +1025,14 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     A.bpp = bpp;
     A.ord = obs_order(bpp, nchunk);
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
-    double* fin = ctx->red + (size_t)nchunk * 2 * g.P;
+    const bool direct = 2 * g.P <= kHostOut;
+    double* fin = direct ? ctx->host_out : ctx->red + (size_t)nchunk * 2 * g.P;
     hipLaunchKernelGGL(k_tmap, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
     hipLaunchKernelGGL(k_tmap_finalize, dim3((unsigned)((2 * g.P + 255) / 256)), dim3(256), 0, ctx->stream, ctx->red,
                        fin, (long)g.P, nchunk);
-    GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if (!direct) GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (direct) std::memcpy(out, fin, 2 * g.P * sizeof(double));
     return 0;
 }
 

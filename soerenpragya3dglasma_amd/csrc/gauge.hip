@@ -758,13 +758,6 @@ int ensure_gauge(glasma_ctx* ctx) {
     return 0;
 }
 
-// host memory for the eight monitors of an iteration and the event that says they are there (kept in the context)
-int ensure_monitors(glasma_ctx* ctx) {
-    if (!ctx->monitors) GL_HIP(ctx, hipHostMalloc(&ctx->monitors, 8 * sizeof(double), hipHostMallocDefault));
-    if (!ctx->monitors_ev) GL_HIP(ctx, hipEventCreateWithFlags(&ctx->monitors_ev, hipEventDisableTiming));
-    return 0;
-}
-
 int ensure_gauge_fixed(glasma_ctx* ctx) {
     if (!ctx->UG) GL_HIP(ctx, hipMalloc(&ctx->UG, (size_t)kUPlanes * pad_sites(ctx->g.S) * sizeof(double)));
     if (!ctx->EG) GL_HIP(ctx, hipMalloc(&ctx->EG, (size_t)kEPlanes * pad_sites(ctx->g.S) * sizeof(double)));
@@ -816,7 +809,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     (void)hipGetLastError();
     const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g, xf);
     rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + 2 * kReduceTmp);
-    if (!rc) rc = ensure_monitors(ctx);
+    if (!rc) rc = ensure_host_out(ctx);
     if (!rc && algo != GLASMA_GAUGE_LOS_ALAMOS) rc = ensure_fftbuf(ctx, 8 * (size_t)g.S);  // 4 complex per site
     if (rc) return rc;
     const double* a = ctx->p.a;
@@ -827,7 +820,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     double* part = ctx->red;                // 2 * nblk blocks of 4 (Los Alamos: both half sweeps)
     double* spart = ctx->red + 8 * nblk;    // step monitors (Los Alamos: both half sweeps)
     double* tmp = ctx->red + 16 * nblk + 8;
-    double* h = ctx->monitors;              // host memory: the reduction writes the eight monitors straight to it
+    double* h = ctx->host_out;              // host memory: the reduction writes the eight monitors straight to it
     double* F = ctx->fftbuf;
     // Los Alamos sweeps read U^G; the Fourier and Jacobi iterations form it on the fly (k_cg_dev_fused) and keep
     // the reference's lag of the top ghost layer by synchronising Gtop right after each deviation kernel, where
@@ -913,14 +906,14 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
         const double mins[2] = {fm0, 0.0};
         reduce_partials(ctx->stream, 2, sets, counts, mins, h, tmp);
         GL_HIP(ctx, hipGetLastError());
-        GL_HIP(ctx, hipEventRecord(ctx->monitors_ev, ctx->stream));
+        GL_HIP(ctx, hipEventRecord(ctx->host_ev, ctx->stream));
         // On small lattices the next iteration's deviation kernel runs while the host reads this one's monitors: it
         // changes nothing that the end of the call uses (not G; Gtop as the end of the call sets it).  That saves 7.5 us
         // an iteration and costs one deviation kernel where the tolerance ends the call: 21 us at 32 x 40 x 64, 85 at
         // 64 x 64 x 128, hence the limit of 512 blocks (131072 sites, about 30 us).
         queued = fused && n + 1 < maxit && nblk <= 512;
         if (queued) deviation();
-        GL_HIP(ctx, hipEventSynchronize(ctx->monitors_ev));
+        GL_HIP(ctx, hipEventSynchronize(ctx->host_ev));
         gmax = h[2];
         gavg = std::sqrt(h[0] / (V * 8.0));
         fmin = h[3];
