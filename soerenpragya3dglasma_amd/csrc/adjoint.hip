@@ -234,18 +234,40 @@ struct DevBuf {
     }
 };
 
-// host charge density (a + 8*Index3D with ghosts) <-> device (a*S + s)
-void rho_to_dev_layout(const glasma_ctx* ctx, const double* h, std::vector<double>& out) {
-    const long S = ctx->g.S, P = ctx->g.P;
-    out.resize(8 * (size_t)S);
-    for (long s = 0; s < S; s++)
-        for (int a = 0; a < 8; a++) out[(size_t)a * S + s] = h[8 * (s + P) + a];
+// host charge density (a + 8*Index3D with ghosts) <-> device (a*S + s), through the field transfers and a tiled array of
+// eight planes (tile, 8 Sp doubles).  The layout change on the host, 2.4 million strided stores and loads at
+// 48 x 48 x 128, and the pageable copies took 3.4 of the 66.7 ms of a gradient call over 100 steps.
+__global__ void k_untile8(const double* __restrict__ tile, double* __restrict__ out, long S) {
+    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= S) return;
+    for (int a = 0; a < 8; a += 2) {
+        const d2_t v = ld2(tile + lidx<long>(8, a, s));
+        out[a * S + s] = v.x;
+        out[(a + 1) * S + s] = v.y;
+    }
 }
-void rho_from_dev_layout(const glasma_ctx* ctx, const std::vector<double>& in, double* h) {
-    const long S = ctx->g.S, P = ctx->g.P;
-    std::memset(h, 0, sizeof(double) * 8 * (size_t)(S + 2 * P));
-    for (long s = 0; s < S; s++)
-        for (int a = 0; a < 8; a++) h[8 * (s + P) + a] = in[(size_t)a * S + s];
+__global__ void k_tile8(const double* __restrict__ in, double* __restrict__ tile, long S) {
+    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= S) return;
+    for (int a = 0; a < 8; a++) tile[lidx<long>(8, a, s)] = in[a * S + s];
+}
+int upload_rho(glasma_ctx* ctx, const double* h, double* rho, double* tile) {
+    const int rc = upload_aos(ctx, h, tile, 8);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_untile8, agrid(ctx->g.S), dim3(kAdjBlock), 0, ctx->stream, tile, rho, ctx->g.S);
+    GL_HIP(ctx, hipGetLastError());
+    return 0;
+}
+int download_rho(glasma_ctx* ctx, const double* rho, double* h, double* tile) {
+    hipLaunchKernelGGL(k_tile8, agrid(ctx->g.S), dim3(kAdjBlock), 0, ctx->stream, rho, tile, ctx->g.S);
+    GL_HIP(ctx, hipGetLastError());
+    const int rc = download_aos(ctx, tile, h, 8);
+    if (rc) return rc;
+    // no charge lives on the ghost layers
+    const size_t layer = 8 * (size_t)ctx->g.P;
+    std::memset(h, 0, sizeof(double) * layer);
+    std::memset(h + 8 * (size_t)ctx->g.S + layer, 0, sizeof(double) * layer);
+    return 0;
 }
 
 bool mv_ok(const glasma_mv_params* mv) { return mv && mv->lambda > 0.0 && mv->m_eff >= 0.0; }
@@ -329,9 +351,7 @@ int glasma_slab_energy_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, 
     tape.V0 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
     tape.V1 = rc ? nullptr : b.get(ctx, 18 * Sp, &rc);
     if (rc) return rc;
-    std::vector<double> h;
-    rho_to_dev_layout(ctx, rho, h);
-    GL_HIP(ctx, hipMemcpy(rho_d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+    if ((rc = upload_rho(ctx, rho, rho_d, tape.V0))) return rc;
     if ((rc = ic_left_from_charge(ctx, mv, rho_d, tape))) return rc;
     for (int n = 0; n < nsteps; n++) {
         launch_step(ctx, n == nsteps - 1);
@@ -431,9 +451,7 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
     if (rc) return rc;
     const bool second = nset > 1 && nrec > 0;  // recomputes go on the second stream
     if (second && (rc = ensure_seg_stream(ctx, nset))) return rc;
-    std::vector<double> h;
-    rho_to_dev_layout(ctx, rho, h);
-    GL_HIP(ctx, hipMemcpy(rho_d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+    if ((rc = upload_rho(ctx, rho, rho_d, tape.V0))) return rc;
     // forward, every step out of place: the segments to recompute from the initial state in the context's fields
     // (left as they are), each checkpoint written by the step that reaches it and the other states alternating between
     // the two tmp states; then the rest into the segment slots, whose sweeps need no recompute
@@ -507,10 +525,7 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
     // the context's fields and UOld still hold the initial state (the linearisation point of the initial-condition
     // map): no step above wrote them
     if ((rc = ic_left_vjp(ctx, mv, tape, cU[cb], cE, cJ[cb], rho_bar, work))) return rc;
-    GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    GL_HIP(ctx, hipMemcpy(h.data(), rho_bar, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    rho_from_dev_layout(ctx, h, grad_rho);
-    return 0;
+    return download_rho(ctx, rho_bar, grad_rho, work);
 }
 
 }  // extern "C"
