@@ -10,7 +10,7 @@
 //
 // The reference walks z sequentially and solves one transverse slice at a time.  Here every transverse
 // operation (charge, smoothing, Poisson solve) runs on all z slices at once as batched 2D FFTs; only the
-// path-ordered Wilson-line product is sequential in z, one thread per transverse site.
+// path-ordered Wilson-line product runs along z, in eight runs side by side.
 //
 // Work arrays (allocated for the call, freed at the end):
 //   F     complex, F[(a*Nz + z)*P + y*Nx + x], a = colour 0..7 (the FFT layout)
@@ -113,24 +113,65 @@ __global__ void k_load_real(double* __restrict__ F, const double* __restrict__ r
     }
 }
 
-// SetNewWilsonLines for all z: one thread per transverse site walks z in the reference's order
-// (L: Nz-1 down to 0 with exp(-i A t / sqrt 2); R: 0 up to Nz-1 with exp(+i A t / sqrt 2)),
-// W <- exp(+-i A(z) t / sqrt 2) W, V(z) = W.
-__global__ void __launch_bounds__(256) k_wilson_scan(const double* __restrict__ F, double* __restrict__ V, Geom g, int right) {
-    long s2 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s2 >= g.P) return;
+// SetNewWilsonLines for all z in the reference's order (L: Nz-1 down to 0 with exp(-i A t / sqrt 2); R: 0 up to Nz-1
+// with exp(+i A t / sqrt 2)): W <- exp(+-i A(z) t / sqrt 2) W, V(z) = W.  The product is cut into runs of z,
+// one wave each, for the block's 64 transverse sites: a run's partial products, then, from the runs' totals in LDS, the
+// product of all earlier runs multiplied in.  One thread per site walking all of z is a serial chain of Nz exponentials on
+// a chip with P / 64 waves: 170 us at 48 x 48 x 128, in eight runs 85.  The runs read and write V once more, so large
+// planes, whose waves fill the chip, take one: 128 x 128 x 256 404 us with one and 375 with eight, 256 x 256 x 128 472
+// and 882.
+constexpr int kScanChunks = 8;
+int scan_chunks(const Geom& g) { return g.P <= 16384 ? kScanChunks : 1; }
+size_t scan_lds(int chunks) { return sizeof(double) * chunks * 18 * 64; }
+__device__ __forceinline__ void st_end(double* ends, int c, const M3& A) {
+    double* const q = ends + (size_t)c * 18 * 64 + (threadIdx.x & 63);
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        q[128 * k] = A.re[k];
+        q[128 * k + 64] = A.im[k];
+    }
+}
+__device__ __forceinline__ void ld_end(const double* ends, int c, M3& A) {
+    const double* const q = ends + (size_t)c * 18 * 64 + (threadIdx.x & 63);
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        A.re[k] = q[128 * k];
+        A.im[k] = q[128 * k + 64];
+    }
+}
+__global__ void __launch_bounds__(64 * kScanChunks) k_wilson_scan(const double* __restrict__ F, double* __restrict__ V,
+                                                                  Geom g, int right) {
+    extern __shared__ double ends[];
+    const int nc = blockDim.x >> 6, c = threadIdx.x >> 6, len = (g.nz + nc - 1) / nc;
+    const long s2 = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int k0 = min(g.nz, c * len), k1 = s2 < g.P ? min(g.nz, k0 + len) : k0;
     M3 W, X, T;
     set_unit(W);
-    const double c = (right ? 1.0 : -1.0) / kSqrt2;
-    for (int k = 0; k < g.nz; k++) {
+    const double cf = (right ? 1.0 : -1.0) / kSqrt2;
+    for (int k = k0; k < k1; k++) {
         const int z = right ? k : g.nz - 1 - k;
         const long s = s2 + g.P * z;
         double col[8];
         for (int a = 0; a < 8; a++) col[a] = F[2 * fidx(g, a, s)];
-        expi(c, col, X);
+        expi(cf, col, X);
         mul_nn(X, W, T);
         W = T;
         stm<long>(V, kGPlanes, 0, s, W);
+    }
+    st_end(ends, c, W);
+    __syncthreads();
+    if (c == 0) return;
+    ld_end(ends, 0, W);
+    for (int j = 1; j < c; j++) {
+        ld_end(ends, j, X);
+        mul_nn(X, W, T);
+        W = T;
+    }
+    for (int k = k0; k < k1; k++) {
+        const long s = s2 + g.P * (right ? k : g.nz - 1 - k);
+        ldm<long>(V, kGPlanes, 0, s, X);
+        mul_nn(X, W, T);
+        stm<long>(V, kGPlanes, 0, s, T);
     }
 }
 
@@ -407,14 +448,16 @@ __global__ void __launch_bounds__(256) k_sheet_sep(const dbl2* __restrict__ A, c
     }
 }
 
-// E_perp(t + dt/2) = MatrixILog(coff_mu, U_mu UOld_mu^dag), E_z = 0 for z in [zlo, zhi]  (:66-92)
+// E_perp(t + dt/2) = MatrixILog(coff_mu, U_mu UOld_mu^dag), E_z = 0 for z in [zlo, zhi]  (:66-92).  Up to 2^19 sites
+// each direction has threads of its own (efield_grid): 8.6 us against 11.6 at 32 x 32 x 32, 106 against 126 at
+// 48 x 48 x 128, but 312 against 291 at 128 x 128 x 128, where one direction's threads fill the chip.
 __global__ void __launch_bounds__(256) k_sheet_efield(const double* __restrict__ U, const double* __restrict__ UO, double* __restrict__ E,
                                Geom g, int zlo, int zhi, double coff0, double coff1) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long n = (long)(zhi - zlo + 1) * g.P;
     if (i >= n) return;
     const long s = i + (long)zlo * g.P;
-    for (int mu = 0; mu < 2; mu++) {
+    for (int mu = blockIdx.y; mu < 2; mu += gridDim.y) {
         M3 A, B, C;
         ldm<long>(U, kUPlanes, 18 * mu, s, A);
         ldm<long>(UO, kUPlanes, 18 * mu, s, B);
@@ -423,6 +466,7 @@ __global__ void __launch_bounds__(256) k_sheet_efield(const double* __restrict__
         ilog(mu == 0 ? coff0 : coff1, C, e);
         stv<long>(E, kEPlanes, 8 * mu, s, e);
     }
+    if (blockIdx.y) return;
     double zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     stv<long>(E, kEPlanes, 16, s, zero);
 }
@@ -593,6 +637,7 @@ __global__ void k_rho_to_aos(const double* __restrict__ rho, double* __restrict_
 }
 
 inline dim3 grid1(long n) { return dim3((unsigned)((n + 255) / 256)); }
+inline dim3 efield_grid(long n) { return dim3(grid1(n).x, n <= (1L << 19) ? 2 : 1); }
 
 int alloc_work(glasma_ctx* ctx, Wk& w) {
     const long S = ctx->g.S, Sp = pad_sites(S);
@@ -623,6 +668,16 @@ void free_work(Wk& w) {
                                                         "prime factors <= 13): ") + fft_last_error()); \
     } while (0)
 
+int wilson_scan(glasma_ctx* ctx, const double* F, double* V, int right) {
+    const int nc = scan_chunks(ctx->g);
+    // the runs' totals are above what a kernel gets without asking
+    GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_wilson_scan),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds(kScanChunks)));
+    hipLaunchKernelGGL(k_wilson_scan, dim3((unsigned)((ctx->g.P + 63) / 64)), dim3(64 * nc), scan_lds(nc), ctx->stream, F, V,
+                       ctx->g, right);
+    return 0;
+}
+
 // Poisson solve of every transverse slice: F (real parts) -> A, imaginary parts of the result dropped
 int poisson_all(glasma_ctx* ctx, double* F) {
     const Geom& g = ctx->g;
@@ -644,7 +699,7 @@ int wilson_from_charge(glasma_ctx* ctx, Wk& w, double lambda, double meff, bool 
     GL_FFT(ctx, fft_xy(ctx->stream, w.F, g, 8, g.nz, +1));
     hipLaunchKernelGGL(k_take_real, grid1(g.S), dim3(256), 0, ctx->stream, w.F, w.rho, g);
     GL_RC(poisson_all(ctx, w.F));
-    hipLaunchKernelGGL(k_wilson_scan, grid1(g.P), dim3(256), 0, ctx->stream, w.F, w.V, g, right ? 1 : 0);
+    GL_RC(wilson_scan(ctx, w.F, w.V, right ? 1 : 0));
     GL_HIP(ctx, hipGetLastError());
     return 0;
 }
@@ -709,13 +764,13 @@ int single_sheet(glasma_ctx* ctx, Wk& w, bool right, int zlo, int zhi, int wstat
     hipLaunchKernelGGL(k_take_real, grid1(g.S), dim3(256), 0, ctx->stream, w.F, (double*)nullptr, g);
     // Wilson lines of the evolved charge (SetWilsonLinesForFirstStep, no smoothing) and U(t + dt) (:40-60)
     GL_RC(poisson_all(ctx, w.F));
-    hipLaunchKernelGGL(k_wilson_scan, grid1(g.P), dim3(256), 0, ctx->stream, w.F, w.V, g, right ? 1 : 0);
+    GL_RC(wilson_scan(ctx, w.F, w.V, right ? 1 : 0));
     hipLaunchKernelGGL(k_sheet_links, grid1(nsl), dim3(256), 0, ctx->stream, w.V, U, g, zlo, zhi);
     // E(t + dt/2) from the logarithm of U UOld^dag (:66-92)
     const double acube = ctx->p.a[0] * ctx->p.a[1] * ctx->p.a[2];
     const double coff0 = -dt * ctx->p.a[0] * ctx->p.a[0] / acube;
     const double coff1 = -dt * ctx->p.a[1] * ctx->p.a[1] / acube;
-    hipLaunchKernelGGL(k_sheet_efield, grid1(nsl), dim3(256), 0, ctx->stream, U, ctx->UOld, ctx->E, g, zlo, zhi, coff0,
+    hipLaunchKernelGGL(k_sheet_efield, efield_grid(nsl), dim3(256), 0, ctx->stream, U, ctx->UOld, ctx->E, g, zlo, zhi, coff0,
                        coff1);
     // J-stat from the transverse Gauss law and J from the z continuity inversion (:98-209)
     SheetSides A;
@@ -953,14 +1008,38 @@ __global__ void __launch_bounds__(256) k_links_vjp(const double* __restrict__ V,
 // Reverse of the left-moving Wilson-line scan V(z) = X(z) V(z+1), X(z) = exp(-i A(z) t / sqrt2), in two kernels.
 // The total cotangent of V(z) is its own Vbar(z) plus, through V(z-1) = X(z-1) V(z), X(z-1)^dag times that of V(z-1);
 // with X(z') ... X(z-1) = V(z') V(z)^dag (V unitary) this is Wbar(z) = V(z) sum_{z' <= z} V(z')^dag Vbar(z'), a running
-// sum along z (k_scan_vjp_sum, one thread per transverse site, Wbar in place of Vbar), after which every layer's
+// sum along z (k_scan_vjp_sum, Wbar in place of Vbar), after which every layer's
 // exponential adjoint is independent (k_scan_vjp_site, one thread per site): Xbar = Wbar(z) V(z+1)^dag.
-__global__ void __launch_bounds__(256) k_scan_vjp_sum(const double* __restrict__ V, double* __restrict__ Vb, Geom g) {
-    long s2 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s2 >= g.P) return;
+// The sum in runs of z as in k_wilson_scan: each run's total, then the walk from the earlier runs' sum; both
+// lines' sums (blockIdx.y) in one launch.  One thread per site took 2 x 225 us at 48 x 48 x 128, the one launch 92.
+struct ScanVjp {
+    const double* V[2];
+    double* Vb[2];
+};
+__global__ void __launch_bounds__(64 * kScanChunks) k_scan_vjp_sum(ScanVjp A, Geom g) {
+    extern __shared__ double ends[];
+    const double* const V = blockIdx.y ? A.V[1] : A.V[0];
+    double* const Vb = blockIdx.y ? A.Vb[1] : A.Vb[0];
+    const int nc = blockDim.x >> 6, c = threadIdx.x >> 6, len = (g.nz + nc - 1) / nc;
+    const long s2 = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int z0 = min(g.nz, c * len), z1 = s2 < g.P ? min(g.nz, z0 + len) : z0;
     M3 acc, Vz, B, T;
     m3_zero(acc);
-    for (int z = 0; z < g.nz; z++) {
+    for (int z = z0; z < z1 && c + 1 < nc; z++) {  // the last run's total is not needed
+        const long s = s2 + g.P * z;
+        ldm<long>(V, kGPlanes, 0, s, Vz);
+        ldm<long>(Vb, kGPlanes, 0, s, B);
+        mul_dn(Vz, B, T);
+        m3_axpy(1.0, T, acc);
+    }
+    st_end(ends, c, acc);
+    __syncthreads();
+    m3_zero(acc);
+    for (int j = 0; j < c; j++) {
+        ld_end(ends, j, T);
+        m3_axpy(1.0, T, acc);
+    }
+    for (int z = z0; z < z1; z++) {
         const long s = s2 + g.P * z;
         ldm<long>(V, kGPlanes, 0, s, Vz);
         ldm<long>(Vb, kGPlanes, 0, s, B);
@@ -1143,7 +1222,7 @@ int ic_left_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, const doubl
     hipLaunchKernelGGL(k_take_real, grid1(g.S), dim3(256), 0, st, F, tape.rho_s, g);
     GL_RC(poisson_all(ctx, F));
     hipLaunchKernelGGL(k_copy_real, grid1(8 * g.S), dim3(256), 0, st, tape.A0, F, g);
-    hipLaunchKernelGGL(k_wilson_scan, grid1(g.P), dim3(256), 0, st, F, tape.V0, g, 0);
+    GL_RC(wilson_scan(ctx, F, tape.V0, 0));
     hipLaunchKernelGGL(k_sheet_links, grid1(g.S), dim3(256), 0, st, tape.V0, ctx->UOld, g, 0, g.nz - 1);
     hipLaunchKernelGGL(k_load_real, grid1(g.S), dim3(256), 0, st, F, tape.rho_s, g);
     GL_FFT(ctx, fft_z(st, F, g, 8, -1));
@@ -1152,12 +1231,12 @@ int ic_left_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, const doubl
     hipLaunchKernelGGL(k_take_real, grid1(g.S), dim3(256), 0, st, F, (double*)nullptr, g);
     GL_RC(poisson_all(ctx, F));
     hipLaunchKernelGGL(k_copy_real, grid1(8 * g.S), dim3(256), 0, st, tape.A1, F, g);
-    hipLaunchKernelGGL(k_wilson_scan, grid1(g.P), dim3(256), 0, st, F, tape.V1, g, 0);
+    GL_RC(wilson_scan(ctx, F, tape.V1, 0));
     hipLaunchKernelGGL(k_sheet_links, grid1(g.S), dim3(256), 0, st, tape.V1, U, g, 0, g.nz - 1);
     const double acube = ctx->p.a[0] * ctx->p.a[1] * ctx->p.a[2];
     const double coff0 = -dt * ctx->p.a[0] * ctx->p.a[0] / acube;
     const double coff1 = -dt * ctx->p.a[1] * ctx->p.a[1] / acube;
-    hipLaunchKernelGGL(k_sheet_efield, grid1(g.S), dim3(256), 0, st, U, ctx->UOld, ctx->E, g, 0, g.nz - 1, coff0, coff1);
+    hipLaunchKernelGGL(k_sheet_efield, efield_grid(g.S), dim3(256), 0, st, U, ctx->UOld, ctx->E, g, 0, g.nz - 1, coff0, coff1);
     SheetSides A;
     A.n = 1;
     A.s[0] = sheet_side(false, 0, g.nz - 1, JPS, JP);
@@ -1203,8 +1282,11 @@ int ic_left_vjp(glasma_ctx* ctx, const glasma_mv_params* mv, const IcTape& tape,
     // links -> Wilson lines -> Poisson solutions
     hipLaunchKernelGGL(k_links_vjp, grid1(g.S), dim3(256), 0, st, tape.V1, Ub, V1b, g);
     hipLaunchKernelGGL(k_links_vjp, grid1(g.S), dim3(256), 0, st, tape.V0, UOb, V0b, g);
-    hipLaunchKernelGGL(k_scan_vjp_sum, grid1(g.P), dim3(256), 0, st, tape.V1, V1b, g);
-    hipLaunchKernelGGL(k_scan_vjp_sum, grid1(g.P), dim3(256), 0, st, tape.V0, V0b, g);
+    const int nc = scan_chunks(g);
+    GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_vjp_sum),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds(kScanChunks)));
+    hipLaunchKernelGGL(k_scan_vjp_sum, dim3((unsigned)((g.P + 63) / 64), 2), dim3(64 * nc), scan_lds(nc), st,
+                       ScanVjp{{tape.V1, tape.V0}, {V1b, V0b}}, g);
     hipLaunchKernelGGL(k_scan_vjp_site, grid1(g.S), dim3(256), 0, st, tape.A1, tape.V1, V1b, A1b, g);
     hipLaunchKernelGGL(k_scan_vjp_site, grid1(g.S), dim3(256), 0, st, tape.A0, tape.V0, V0b, A0b, g);
     // rho_ev cotangent = poisson(A1bar); rho_s cotangent = evolve_R(that) + poisson(A0bar)
