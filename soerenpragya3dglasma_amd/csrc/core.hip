@@ -34,12 +34,6 @@ int ensure_red(glasma_ctx* ctx, size_t doubles) {
     ctx->red_cap = doubles;
     return 0;
 }
-// the host memory for small results and its event (kept in the context)
-int ensure_host_out(glasma_ctx* ctx) {
-    if (!ctx->host_out) GL_HIP(ctx, hipHostMalloc(&ctx->host_out, kHostOut * sizeof(double), hipHostMallocDefault));
-    if (!ctx->host_ev) GL_HIP(ctx, hipEventCreateWithFlags(&ctx->host_ev, hipEventDisableTiming));
-    return 0;
-}
 int ensure_fftbuf(glasma_ctx* ctx, size_t doubles) {
     if (ctx->fftbuf_cap >= doubles) return 0;
     if (ctx->fftbuf) (void)hipFree(ctx->fftbuf);
@@ -629,7 +623,6 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     const Geom& g = ctx->g;
     const int bpp = (int)((g.P + 255) / 256);
     int rc = ensure_red(ctx, (size_t)g.nz * bpp * K + (size_t)g.nz * K);
-    if (!rc) rc = ensure_host_out(ctx);
     if (rc) return rc;
     ObsArgs A;
     A.U = ctx->U[ctx->cur];
@@ -710,6 +703,8 @@ int glasma_create(const glasma_params* p, glasma_ctx** out) {
     if (e == hipSuccess) e = hipMalloc(&ctx->E, (size_t)kEPlanes * S * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&ctx->J[0], (size_t)kJPlanes * S * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&ctx->J[1], (size_t)kJPlanes * S * sizeof(double));
+    if (e == hipSuccess) e = hipHostMalloc(&ctx->host_out, kHostOut * sizeof(double), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->host_ev, hipEventDisableTiming);
     if (e != hipSuccess) {
         const int code = hip_code(e);
         glasma_destroy(ctx);
@@ -1013,7 +1008,6 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     const int bpp = (int)((g.P + 255) / 256);
     const int chunk = map_chunk(g), nchunk = (g.nz + chunk - 1) / chunk;
     int rc = ensure_red(ctx, (size_t)(nchunk + 1) * 2 * g.P);
-    if (!rc) rc = ensure_host_out(ctx);
     if (rc) return rc;
     ObsArgs A;
     A.U = ctx->U[ctx->cur];

@@ -809,7 +809,6 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     (void)hipGetLastError();
     const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g, xf);
     rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + 2 * kReduceTmp);
-    if (!rc) rc = ensure_host_out(ctx);
     if (!rc && algo != GLASMA_GAUGE_LOS_ALAMOS) rc = ensure_fftbuf(ctx, 8 * (size_t)g.S);  // 4 complex per site
     if (rc) return rc;
     const double* a = ctx->p.a;

@@ -70,7 +70,8 @@ struct glasma_ctx {
     // recompute there overlaps the previous segment's backward sweep
     hipStream_t stream2 = nullptr;
     std::vector<hipEvent_t> seg_ev;
-    // pinned host memory that kernels write small results to (kHostOut doubles), and an event to wait for them
+    // pinned host memory that kernels write small results to (kHostOut doubles; pinning it takes about 60 us, so it is
+    // made with the context), and an event to wait for them
     double* host_out = nullptr;
     hipEvent_t host_ev = nullptr;
     std::string err;
@@ -86,7 +87,6 @@ int hip_fail(glasma_ctx* ctx, hipError_t e, const char* what);
 int hip_code(hipError_t e);
 int ensure_red(glasma_ctx* ctx, size_t doubles);
 constexpr long kHostOut = 8192;
-int ensure_host_out(glasma_ctx* ctx);
 int ensure_fftbuf(glasma_ctx* ctx, size_t doubles);
 int reset_fields(glasma_ctx* ctx);
 // host array in the reference AoS layout with z ghosts (R doubles per site) <-> planes p0..p0+R-1 of a
