@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("driver,N", [(0, (11, 13, 9)), (1, (72, 75, 3)), (0, (72, 75, 4)), (2, (4, 3, 600)),
-                                      (0, (3, 5, 2048)), (0, (5, 7, 1)), (2, (1, 6, 10)), (0, (64, 64, 6))])
+                                      (0, (3, 5, 2048)), (0, (5, 7, 1)), (2, (1, 6, 10)), (0, (64, 64, 6)), (1, (56, 88, 4))])
 def test_sheet_shapes(driver, N):
     from soerenpragya3dglasma_amd import Glasma
     a, dt = (1.0, 0.9, 1.1), 0.25
