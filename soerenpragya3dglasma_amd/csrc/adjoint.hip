@@ -127,6 +127,7 @@ int slab_energy(glasma_ctx* ctx, int zc, int half, double* out, const double* U 
     if (E) A.E = E;
     hipLaunchKernelGGL(k_slab_energy, dim3((unsigned)nb), dim3(kAdjBlock), 0, ctx->stream, A, ctx->red);
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kAdjBlock), 0, ctx->stream, ctx->red, nb, ctx->red + nb);
+    GL_HIP(ctx, hipGetLastError());
     GL_HIP(ctx, hipMemcpyAsync(out, ctx->red + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return 0;

@@ -643,6 +643,7 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     double* fin = direct ? ctx->host_out : ctx->red + (size_t)g.nz * bpp * K;
     hipLaunchKernelGGL(k_finalize, dim3((n + kFinOuts - 1) / kFinOuts), dim3(64 * kFinOuts), 0, ctx->stream, ctx->red, fin,
                        g.nz, bpp, K, maxmask);
+    GL_HIP(ctx, hipGetLastError());  // before the result is read: host_out still holds the previous record's
     per_z.resize(n);
     if (!direct)
         GL_HIP(ctx, hipMemcpyAsync(per_z.data(), fin, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1024,6 +1025,7 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     hipLaunchKernelGGL(k_tmap, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
     hipLaunchKernelGGL(k_tmap_finalize, dim3((unsigned)((2 * g.P + 255) / 256)), dim3(256), 0, ctx->stream, ctx->red,
                        fin, (long)g.P, nchunk);
+    GL_HIP(ctx, hipGetLastError());
     if (!direct) GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (direct) std::memcpy(out, fin, 2 * g.P * sizeof(double));

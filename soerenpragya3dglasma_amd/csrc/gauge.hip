@@ -970,6 +970,7 @@ extern "C" int glasma_gauss_restore(glasma_ctx* ctx, int transverse_only, double
     };
     double h[4];
     auto read = [&]() -> int {
+        GL_HIP(ctx, hipGetLastError());
         GL_HIP(ctx, hipMemcpyAsync(h, fin, 4 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
         return 0;
@@ -983,7 +984,6 @@ extern "C" int glasma_gauss_restore(glasma_ctx* ctx, int transverse_only, double
             deviation();
             hipLaunchKernelGGL(k_gr_efield, grid1(g.S), dim3(kCgBlock), 0, ctx->stream, U, ctx->E, Gv, g, gammas[k], nmu);
         }
-        GL_HIP(ctx, hipGetLastError());
         if ((rc = read())) return rc;  // the violation of the third step, measured before its update
         n++;
     }

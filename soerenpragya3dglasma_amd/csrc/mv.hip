@@ -1427,8 +1427,10 @@ extern "C" int glasma_set_wilson_lines(glasma_ctx* ctx, char dir, const glasma_m
         hipError_t e = hipMalloc(&tmp, 8 * (size_t)g.S * sizeof(double));
         if (e == hipSuccess) {
             hipLaunchKernelGGL(k_rho_to_aos, grid1(8 * g.S), dim3(256), 0, ctx->stream, w.rho, tmp, g);
-            e = hipMemcpyAsync(rho_out + 8 * g.P, tmp, 8 * (size_t)g.S * sizeof(double), hipMemcpyDeviceToHost,
-                               ctx->stream);
+            e = hipGetLastError();
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(rho_out + 8 * g.P, tmp, 8 * (size_t)g.S * sizeof(double), hipMemcpyDeviceToHost,
+                                   ctx->stream);
             if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
             (void)hipFree(tmp);
         }
