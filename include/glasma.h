@@ -313,14 +313,18 @@ int glasma_step_vjp(glasma_ctx* ctx, double* Ub, double* Eb, double* Jpb, double
 int glasma_slab_energy_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, const double* rho, int nsteps, int zc,
                                    int half, double* energy);
 /* The same energy and its gradient with respect to rho (grad_rho: same layout, ghosts zero), by
- * reverse-mode differentiation of the steps (forward states checkpointed every ckpt steps; the last segments, as many
- * as a quarter of the device memory and half of the free memory hold, are kept whole, each earlier one is recomputed
- * once) and of the initial conditions.  The context holds the initial state afterwards.  Both calls keep
- * their device work arrays in the context (counted by glasma_memory_bytes, freed by glasma_destroy), so that
- * repeated calls of one size allocate nothing.  When memory allows, a segment's recompute runs on a second stream
- * of the context (created on first use, default priority) beside the backward sweep; the call returns after both. */
+ * reverse-mode differentiation of the steps (forward states checkpointed every ckpt steps; the last two segments are
+ * kept whole, or as many as glasma_set_gradient_memory allows, each earlier one is recomputed once) and of the initial
+ * conditions.  The context holds the initial state afterwards.  Both calls keep their device work arrays in the context
+ * (counted by glasma_memory_bytes, freed by glasma_destroy and by glasma_set_gradient_memory), so that repeated calls
+ * of one size allocate nothing.  When memory allows, a segment's recompute runs on a second stream of the context (created on first use, default priority) beside the backward sweep; the call returns after both. */
 int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, const double* rho, int nsteps, int ckpt,
                                 int zc, int half, double* energy, double* grad_rho);
+/* Memory that the gradient call may hold for segments kept whole instead of recomputed: sets of ckpt states, each
+ * ckpt * 1312 bytes per site, as many as fit `bytes` (at least one; never more than a quarter of the device memory and
+ * half of what is free).  0, the default: two sets, so that ckpt alone decides.  Gives back the work arrays that the
+ * context holds. */
+int glasma_set_gradient_memory(glasma_ctx* ctx, size_t bytes);
 
 /* ---- per-site SU(3) algebra on the device, batched (tests and tools) ------------------------- */
 /* op: 0 exp(i c alpha t) [in: n*8 alpha, out: n*18], 1 log [in: n*18 U, out: n*8],

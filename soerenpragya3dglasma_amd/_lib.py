@@ -113,6 +113,7 @@ def lib():
         "glasma_step_vjp": ([vp] + [dp] * 6, c_int),
         "glasma_slab_energy_from_charge": ([vp, ctypes.POINTER(MVParams), dp, c_int, c_int, c_int, dp], c_int),
         "glasma_slab_energy_gradient": ([vp, ctypes.POINTER(MVParams), dp, c_int, c_int, c_int, c_int, dp, dp], c_int),
+        "glasma_set_gradient_memory": ([vp, ctypes.c_size_t], c_int),
     }
     for name, (args, res) in sig.items():
         fn = getattr(L, name, None)

@@ -1,8 +1,8 @@
 // Reverse-mode derivatives on the device (no counterpart in the reference, which has no gradient code):
 // the leapfrog step (two passes per step, no atomics: A with B folded in, then the staple gather), the slab
 // energy, and the whole map charge density -> left-moving MV sheet -> nsteps leapfrog steps -> slab energy, with
-// the forward run checkpointed every ckpt steps: the last segments, as many as the memory holds, are kept whole, each
-// earlier one is recomputed once during the backward sweep.
+// the forward run checkpointed every ckpt steps: the last segments (two, or as many as the caller's limit holds) are kept
+// whole, each earlier one is recomputed once during the backward sweep.
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -235,6 +235,14 @@ struct DevBuf {
     }
 };
 
+// gives the pool's arrays back, once nothing queued uses them
+void free_work_pool(glasma_ctx* ctx) {
+    (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->stream2) (void)hipStreamSynchronize(ctx->stream2);
+    for (auto& p : ctx->wpool) (void)hipFree(p.second);
+    ctx->wpool.clear();
+}
+
 // host charge density (a + 8*Index3D with ghosts) <-> device (a*S + s), through the field transfers and a tiled array of
 // eight planes (tile, 8 Sp doubles).  The layout change on the host, 2.4 million strided stores and loads at
 // 48 x 48 x 128, and the pageable copies took 3.4 of the 66.7 ms of a gradient call over 100 steps.
@@ -363,6 +371,13 @@ int glasma_slab_energy_from_charge(glasma_ctx* ctx, const glasma_mv_params* mv, 
     return slab_energy(ctx, zc, half, energy);
 }
 
+int glasma_set_gradient_memory(glasma_ctx* ctx, size_t bytes) {
+    if (!ctx) return GLASMA_ERR_ARG;
+    ctx->grad_bytes = bytes;
+    free_work_pool(ctx);
+    return 0;
+}
+
 int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, const double* rho, int nsteps, int ckpt,
                                 int zc, int half, double* energy, double* grad_rho) {
     if (!ctx || !rho || !energy || !grad_rho || nsteps < 0 || ckpt <= 0 || half < 0 || !mv_ok(mv)) return GLASMA_ERR_ARG;
@@ -373,23 +388,26 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
     // The segment slots are kept in nset sets (segment sg uses set sg % nset).  The forward run leaves the states of the
     // last nset segments in them; an earlier segment starts from a checkpoint and is recomputed into its set, on the
     // second stream, once the sweep over the segment that held the set is done, beside the sweeps of the segments in
-    // between.  As many sets as a quarter of the device memory holds (two where one takes no more than that quarter,
-    // one beyond): a recomputed step costs a forward step, so the gradient of 100 steps with checkpoints every 20 at
-    // 48 x 48 x 128 took 78 ms with four of five segments recomputed, 77, 73 and 70 with two, three and four
-    // kept and 67 with all five (38 GB).
+    // between.  Two sets, so that ckpt decides what the call holds (one where a set takes more than a quarter of the
+    // device memory); as many as fit its limit when the caller has set one (glasma_set_gradient_memory), within a quarter
+    // of the device memory and half of what is free.  A recomputed step costs a forward step: the gradient of 100 steps with
+    // checkpoints every 20 at 48 x 48 x 128 took 78 ms with one of five segments kept, 74 with two, 69 with four and 64.5
+    // with all five (38 GB).
     int nset = 1, nset0 = 1;  // nset0: without the sets beyond two
     if (nseg > 1) {
         size_t freeb = 0, totalb = 0, held = 0;
         for (const auto& p : ctx->wpool) held += p.first * sizeof(double);
         const size_t set_bytes = (size_t)seglen * (2 * kUPlanes + kEPlanes + kJPlanes) * Sp * sizeof(double);
+        size_t want = ctx->grad_bytes ? std::max<size_t>(1, ctx->grad_bytes / set_bytes) : 2;
+        const char* env = std::getenv("GLASMA_GRAD_SETS");  // that many sets in place of either (read on every call)
+        if (env && std::atoi(env) >= 1) want = std::atoi(env);
         if (hipMemGetInfo(&freeb, &totalb) == hipSuccess) {
-            if (set_bytes <= totalb / 4) nset = 2;
+            if (set_bytes <= totalb / 4 && want >= 2) nset = 2;
             nset0 = nset;
-            while (nset < nseg && (size_t)(nset + 1) * set_bytes <= std::min(totalb / 4, (freeb + held) / 2)) nset++;
+            while (nset < nseg && (size_t)nset < want &&
+                   (size_t)(nset + 1) * set_bytes <= std::min(totalb / 4, (freeb + held) / 2))
+                nset++;
         }
-        const char* env = std::getenv("GLASMA_GRAD_SETS");  // that many sets at most (read on every call)
-        if (env && std::atoi(env) >= 1) nset = std::min(nset, std::atoi(env));
-        nset0 = std::min(nset0, nset);
     }
     int nrec = 0;  // segments to recompute: the first nrec
     IcTape tape;
@@ -442,9 +460,7 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
     allocate();
     if (rc && nset > nset0) {  // another user took the memory meanwhile: without the extra sets
         (void)hipGetLastError();
-        (void)hipStreamSynchronize(ctx->stream);
-        for (auto& p : ctx->wpool) (void)hipFree(p.second);
-        ctx->wpool.clear();
+        free_work_pool(ctx);
         nset = nset0;
         rc = 0;
         allocate();

@@ -66,6 +66,7 @@ struct glasma_ctx {
     // work arrays of the slab-energy and gradient calls (doubles, pointer), handed out in request order and kept for
     // the next call, so that repeated calls of one size allocate nothing; freed by glasma_destroy
     std::vector<std::pair<size_t, double*>> wpool;
+    size_t grad_bytes = 0;  // limit of the gradient's segment sets (glasma_set_gradient_memory); 0: two sets
     // second stream and events of the gradient call (created on first use, default priority): a checkpoint segment's
     // recompute there overlaps the previous segment's backward sweep
     hipStream_t stream2 = nullptr;

@@ -383,6 +383,11 @@ class Glasma:
                   "glasma_slab_energy_gradient")
         return e.value, gr[1:-1].copy()
 
+    def set_gradient_memory(self, nbytes: int):
+        """Device memory that slab_energy_gradient may hold for segments kept whole instead of recomputed, 1312 bytes per
+        site and step (0, the default: two segments of ckpt steps).  Gives back the work arrays held so far."""
+        self._chk(_lib.lib().glasma_set_gradient_memory(self._h, int(nbytes)), "glasma_set_gradient_memory")
+
     # -- gauge fixing -------------------------------------------------------------------------------
     def coulomb_gauge(self, tol: float = 1e-15, maxit: int = 1000, alpha: float = 2.0) -> np.ndarray:
         stats = np.zeros(7)
