@@ -457,13 +457,14 @@ int glasma_slab_energy_gradient(glasma_ctx* ctx, const glasma_mv_params* mv, con
         rho_bar = rc ? nullptr : b.get(ctx, 8 * S, &rc);
         work = rc ? nullptr : b.get(ctx, 54 * Sp + 36 * Sp + 32 * S, &rc);
     };
+    const std::string said = ctx->err;
     allocate();
     if (rc && nset > nset0) {  // another user took the memory meanwhile: without the extra sets
-        (void)hipGetLastError();
         free_work_pool(ctx);
         nset = nset0;
         rc = 0;
         allocate();
+        if (!rc) ctx->err = said;
     }
     if (rc) return rc;
     const bool second = nset > 1 && nrec > 0;  // recomputes go on the second stream

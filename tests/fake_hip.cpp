@@ -13,7 +13,7 @@ namespace {
 std::mutex mu;
 std::map<void*, size_t> device, pinned;
 long launches, refuse = -1, streams, pins, transfers_h2d, transfers_d2h;
-size_t limit = (size_t)288 << 30, used, pin_limit = ~(size_t)0, pinned_bytes;
+size_t limit = (size_t)288 << 30, shown, used, pin_limit = ~(size_t)0, pinned_bytes;
 thread_local hipError_t last = hipSuccess;
 hipError_t fail(hipError_t e) { return last = e; }
 hipError_t get(std::map<void*, size_t>& m, size_t& total, size_t cap, void** p, size_t n) {
@@ -57,6 +57,7 @@ extern "C" {
 // controls
 void fake_refuse_launch(long n) { refuse = n < 0 ? -1 : launches + n; }  // the n-th launch from now on
 void fake_limit(size_t bytes) { limit = bytes; }
+void fake_show(size_t bytes) { shown = bytes; }  // what hipMemGetInfo calls the device's memory (0: the limit)
 void fake_pin_limit(size_t bytes) { pin_limit = bytes; }
 long fake_launches() { return launches; }
 long fake_streams() { return streams; }
@@ -75,8 +76,8 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
 hipError_t hipHostFree(void* p) { return put(pinned, pinned_bytes, p); }
 hipError_t hipMemGetInfo(size_t* f, size_t* t) {
     std::lock_guard<std::mutex> lock(mu);
-    *t = limit;
-    *f = limit > used ? limit - used : 0;
+    *t = shown ? shown : limit;
+    *f = *t > used ? *t - used : 0;
     return hipSuccess;
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) { return copy(d, s, n, k); }

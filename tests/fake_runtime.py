@@ -14,7 +14,7 @@ for f in ("launches", "streams", "pins", "copies"):
 for f in ("used", "pinned"):
     getattr(fake, "fake_" + f).restype = ctypes.c_size_t
 fake.fake_refuse_launch.argtypes = [ctypes.c_long]
-fake.fake_limit.argtypes = fake.fake_pin_limit.argtypes = [ctypes.c_size_t]
+fake.fake_limit.argtypes = fake.fake_show.argtypes = fake.fake_pin_limit.argtypes = [ctypes.c_size_t]
 sys.path.insert(0, {root!r})
 import numpy as np
 from soerenpragya3dglasma_amd import Glasma, GlasmaBatch, GlasmaError, _lib

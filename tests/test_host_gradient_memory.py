@@ -48,3 +48,45 @@ g.close()
 
 def test_gradient_memory_follows_ckpt():
     fake_runtime.run(SCRIPT)
+
+
+FALLBACK = """
+N, steps, ckpt = (8, 8, 16), 40, 2
+S = N[0] * N[1] * N[2]
+xl, _ = Glasma.draw_charges(1, N[0], N[1], 0.5, 0.5)
+mv = Glasma.mv_params(1.65, 0.1, 2.0, 2.0, 5, 9)
+rho = np.zeros((N[2], N[1], N[0], 8))
+g = Glasma(N)
+for message in (False, True):
+    if message:  # a message that an earlier call left
+        assert _lib.lib().glasma_set_wilson_lines(g._h, b"X", ctypes.byref(mv), None, None, None) != 0
+    before = _lib.lib().glasma_last_error(g._h)
+    assert bool(before) == message
+    g.slab_energy_gradient(mv, rho, steps, ckpt, 8, 4)
+    need = fake.fake_used()  # with two sets
+    g.set_gradient_memory(1 << 40)
+    fake.fake_show(288 << 30)
+    fake.fake_limit(need + 8 * S * 3 * ckpt * 164)  # three sets more, though the device seems to have room for all
+    for _ in range(2):
+        g.slab_energy_gradient(mv, rho, steps, ckpt, 8, 4)
+        assert _lib.lib().glasma_last_error(g._h) == before, _lib.lib().glasma_last_error(g._h)
+        assert fake.fake_used() <= need
+    g.set_gradient_memory(0)
+    fake.fake_limit(need // 2)  # not even the two sets: an error
+    try:
+        g.slab_energy_gradient(mv, rho, steps, ckpt, 8, 4)
+    except GlasmaError as e:
+        assert "allocation" in str(e)
+    else:
+        raise SystemExit("no error")
+    fake.fake_limit(288 << 30)
+    fake.fake_show(0)
+    g.close()
+    g = Glasma(N)
+"""
+
+
+def test_fallback_to_two_sets_leaves_no_message():
+    """When another user of the device takes the memory that seemed free, the call goes on with two sets, and
+    glasma_last_error keeps what it said before."""
+    fake_runtime.run(FALLBACK)
