@@ -59,6 +59,7 @@ def lib():
         "glasma_destroy": ([vp], c_int),
         "glasma_last_error": ([vp], ctypes.c_char_p),
         "glasma_version": ([], ctypes.c_char_p),
+        "glasma_release_idle": ([], c_int),
         "glasma_memory_bytes": ([vp, ctypes.POINTER(ctypes.c_size_t)], c_int),
         "glasma_set_fields": ([vp] + [dp] * 6, c_int),
         "glasma_get_fields": ([vp] + [dp] * 6, c_int),

@@ -745,6 +745,11 @@ int glasma_destroy(glasma_ctx* ctx) {
     return 0;
 }
 
+int glasma_release_idle(void) {
+    stage_release_idle();
+    return 0;
+}
+
 int glasma_memory_bytes(const glasma_ctx* ctx, size_t* bytes) {
     if (!ctx || !bytes) return GLASMA_ERR_ARG;
     const size_t S = ctx->g.S;

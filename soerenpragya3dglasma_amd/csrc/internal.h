@@ -97,6 +97,7 @@ int download_aos(glasma_ctx* ctx, const double* dev_soa, double* host_with_ghost
 // the process's contexts, for the transfers' pinned buffers (transfer.hip)
 void stage_context_created();
 void stage_context_destroyed();
+void stage_release_idle();
 void host_sync_ghosts(const glasma_ctx* ctx, double* h, int R);
 __global__ void k_set_identity(double* __restrict__ U, long S, int nmat);
 

@@ -9,9 +9,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "internal.h"
@@ -22,7 +22,6 @@ namespace {
 
 constexpr size_t kPiece = 1 << 20;
 constexpr int kWorkers = 8;
-constexpr int kIdleSets = 2;
 
 // the pinned buffers and streams of one transfer
 struct StageSet {
@@ -31,8 +30,13 @@ struct StageSet {
     hipStream_t stream[kWorkers] = {};
 };
 
-// Sets not in use, at most kIdleSets of them, kept until the process holds no context any more: pinning 8 MiB takes longer
-// than a small transfer.
+// Sets not in use: at most kIdleSets (for that many threads at once) while the process holds contexts, one after that,
+// until glasma_release_idle.  A set costs 2 to 12 ms to make and give back (pinning 8 MiB, eight streams), more than small
+// fields take, so contexts made one after another and threads side by side have to find theirs again.  A context with its
+// fields set and read took 2.8 ms at 16 x 16 x 32 and 13.6 to 16 at 32 x 32 x 64 when the last context took the sets with
+// it (1.8 and 13.4 through the runtime's own staging), 1.05 and 7.5 now; eight threads with two idle sets between them 0.69
+// ms for set and get at 16 x 16 x 32, 0.35 now.
+constexpr int kIdleSets = 8;
 std::mutex g_mu;
 StageSet* g_idle[kIdleSets] = {};
 int g_contexts = 0;
@@ -45,8 +49,8 @@ void destroy_set(StageSet* s) {
     delete s;
 }
 
-// a set for the current device with the buffers of the first `workers` workers
-hipError_t acquire_set(int device, int workers, StageSet** out) {
+// a set for the current device with the buffers of up to *workers workers (fewer where no more memory can be pinned)
+hipError_t acquire_set(int device, int* workers, StageSet** out) {
     StageSet* s = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_mu);
@@ -59,14 +63,18 @@ hipError_t acquire_set(int device, int workers, StageSet** out) {
         s->device = device;
     }
     hipError_t e = hipSuccess;
-    for (int w = 0; w < workers && e == hipSuccess; w++) {
-        if (!s->buf[w]) e = hipHostMalloc(reinterpret_cast<void**>(&s->buf[w]), kPiece, hipHostMallocDefault);
-        if (e == hipSuccess && !s->stream[w]) e = hipStreamCreate(&s->stream[w]);
+    int n = 0;
+    for (; n < *workers; n++) {
+        if (!s->buf[n]) e = hipHostMalloc(reinterpret_cast<void**>(&s->buf[n]), kPiece, hipHostMallocDefault);
+        if (e == hipSuccess && !s->stream[n]) e = hipStreamCreate(&s->stream[n]);
+        if (e != hipSuccess) break;
     }
-    if (e != hipSuccess) {
+    if (n == 0) {
         destroy_set(s);
         return e;
     }
+    if (e != hipSuccess) (void)hipGetLastError();
+    *workers = n;
     *out = s;
     return hipSuccess;
 }
@@ -115,12 +123,12 @@ int transfer(glasma_ctx* ctx, double* host, double* soa, int R, int NP, int p0) 
     const long npiece = (S + per - 1) / per;
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const unsigned hc = std::thread::hardware_concurrency();
-    const int workers = (int)std::min<long>(npiece, std::min<long>(kWorkers, hc > 2 ? hc : 2));
+    int workers = (int)std::min<long>(npiece, std::min<long>(kWorkers, hc > 2 ? hc : 2));
     int current = ctx->device;
     GL_HIP(ctx, hipGetDevice(&current));
     if (current != ctx->device) GL_HIP(ctx, hipSetDevice(ctx->device));
     StageSet* set = nullptr;
-    hipError_t e0 = acquire_set(ctx->device, workers, &set);
+    hipError_t e0 = acquire_set(ctx->device, &workers, &set);
     if (e0 != hipSuccess) {
         if (current != ctx->device) (void)hipSetDevice(current);
         return hip_fail(ctx, e0, "pinned buffers of a field transfer");
@@ -146,16 +154,18 @@ int transfer(glasma_ctx* ctx, double* host, double* soa, int R, int NP, int p0) 
     for (int w = 1; w < workers; w++) {
         try {
             th[w] = std::thread(work, w);
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {
             break;  // the workers that run take its pieces
         }
     }
     work(0);
     for (std::thread& t : th)
         if (t.joinable()) t.join();
+    const hipError_t e = (hipError_t)failed.load();
+    if (e != hipSuccess)  // a kernel may still be using a buffer
+        for (int w = 0; w < workers; w++) (void)hipStreamSynchronize(set->stream[w]);
     release_set(set);
     if (current != ctx->device) (void)hipSetDevice(current);
-    const hipError_t e = (hipError_t)failed.load();
     if (e != hipSuccess) return hip_fail(ctx, e, TO_DEVICE ? "upload_aos" : "download_aos");
     return 0;
 }
@@ -166,15 +176,26 @@ void stage_context_created() {
     std::lock_guard<std::mutex> lock(g_mu);
     g_contexts++;
 }
-void stage_context_destroyed() {
+// gives the sets not in use back, all but `keep` of them
+static void release_idle(int keep) {
     StageSet* gone[kIdleSets] = {};
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        if (--g_contexts == 0) std::swap(gone, g_idle);
+        for (int i = 0; i < kIdleSets; i++)
+            if (g_idle[i] && keep-- <= 0) std::swap(gone[i], g_idle[i]);
     }
     for (StageSet* s : gone)
         if (s) destroy_set(s);
 }
+void stage_context_destroyed() {
+    bool last;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        last = --g_contexts == 0;
+    }
+    if (last) release_idle(1);
+}
+void stage_release_idle() { release_idle(0); }
 
 int upload_aos(glasma_ctx* ctx, const double* host_with_ghosts, double* dev_soa, int R, int NP, int p0) {
     return transfer<true>(ctx, const_cast<double*>(host_with_ghosts) + (size_t)ctx->g.P * R, dev_soa, R, NP < 0 ? R : NP, p0);

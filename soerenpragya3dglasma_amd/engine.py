@@ -512,6 +512,11 @@ class GlasmaBatch:
         self.close()
 
 
+def release_idle():
+    """Give back the pinned host memory and the streams kept for the field transfers of the next lattice."""
+    _lib.lib().glasma_release_idle()
+
+
 def fft_host(data: np.ndarray, dims, batch: int, sign: int) -> np.ndarray:
     """Device FFT of a host complex array (FFTW conventions, unnormalised)."""
     d = np.ascontiguousarray(data, np.complex128).copy()
