@@ -73,8 +73,8 @@ int glasma_create(const glasma_params* p, glasma_ctx** out);
 int glasma_destroy(glasma_ctx* ctx);
 const char* glasma_last_error(const glasma_ctx* ctx);   /* ctx may be NULL (creation errors) */
 const char* glasma_version(void);
-/* Gives back the pinned host memory (8 MiB at most once no context is left) and the streams that the library keeps for
- * the field transfers of the next context. */
+/* Gives back the pinned host memory (8 MiB and 64 KiB at most once no context is left) and the streams that the library
+ * keeps for the field transfers and records of the next context. */
 int glasma_release_idle(void);
 /* device bytes held by the context */
 int glasma_memory_bytes(const glasma_ctx* ctx, size_t* bytes);

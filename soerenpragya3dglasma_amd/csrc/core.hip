@@ -639,15 +639,17 @@ static int run_obs(glasma_ctx* ctx, void (*kern)(ObsArgs), int K, unsigned maxma
     // results that fit go straight to pinned host memory: a copy to pageable memory is a launch, a staging copy and their
     // gaps (six records of 64 x 56 x 96 took 528 us with the copies and 472 without)
     const int n = g.nz * K;
-    const bool direct = n <= kHostOut;
-    double* fin = direct ? ctx->host_out : ctx->red + (size_t)g.nz * bpp * K;
+    HostOut out(ctx, n);
+    const bool direct = out.p != nullptr;
+    double* fin = direct ? out.p : ctx->red + (size_t)g.nz * bpp * K;
     hipLaunchKernelGGL(k_finalize, dim3((n + kFinOuts - 1) / kFinOuts), dim3(64 * kFinOuts), 0, ctx->stream, ctx->red, fin,
                        g.nz, bpp, K, maxmask);
-    GL_HIP(ctx, hipGetLastError());  // before the result is read: host_out still holds the previous record's
+    GL_HIP(ctx, hipGetLastError());  // before the result is read: the memory still holds a previous record's
     per_z.resize(n);
     if (!direct)
         GL_HIP(ctx, hipMemcpyAsync(per_z.data(), fin, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    out.busy = false;
     if (direct) std::memcpy(per_z.data(), fin, n * sizeof(double));
     return 0;
 }
@@ -704,7 +706,6 @@ int glasma_create(const glasma_params* p, glasma_ctx** out) {
     if (e == hipSuccess) e = hipMalloc(&ctx->E, (size_t)kEPlanes * S * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&ctx->J[0], (size_t)kJPlanes * S * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&ctx->J[1], (size_t)kJPlanes * S * sizeof(double));
-    if (e == hipSuccess) e = hipHostMalloc(&ctx->host_out, kHostOut * sizeof(double), hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->host_ev, hipEventDisableTiming);
     if (e != hipSuccess) {
         const int code = hip_code(e);
@@ -734,7 +735,6 @@ int glasma_destroy(glasma_ctx* ctx) {
         if (w.second) (void)hipFree(w.second);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
-    if (ctx->host_out) (void)hipHostFree(ctx->host_out);
     if (ctx->host_ev) hipEventDestroy(ctx->host_ev);
     for (hipEvent_t ev : ctx->seg_ev)
         if (ev) hipEventDestroy(ev);
@@ -1025,14 +1025,16 @@ int glasma_transverse_energy_map(glasma_ctx* ctx, double* out) {
     A.bpp = bpp;
     A.ord = obs_order(bpp, nchunk);
     for (int m = 0; m < 3; m++) A.a[m] = ctx->p.a[m];
-    const bool direct = 2 * g.P <= kHostOut;
-    double* fin = direct ? ctx->host_out : ctx->red + (size_t)nchunk * 2 * g.P;
+    HostOut host(ctx, 2 * g.P);
+    const bool direct = host.p != nullptr;
+    double* fin = direct ? host.p : ctx->red + (size_t)nchunk * 2 * g.P;
     hipLaunchKernelGGL(k_tmap, dim3((unsigned)(A.ord.per * kXcds)), dim3(256), 0, ctx->stream, A, ctx->red, chunk);
     hipLaunchKernelGGL(k_tmap_finalize, dim3((unsigned)((2 * g.P + 255) / 256)), dim3(256), 0, ctx->stream, ctx->red,
                        fin, (long)g.P, nchunk);
     GL_HIP(ctx, hipGetLastError());
     if (!direct) GL_HIP(ctx, hipMemcpyAsync(out, fin, 2 * g.P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    host.busy = false;
     if (direct) std::memcpy(out, fin, 2 * g.P * sizeof(double));
     return 0;
 }

@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <cstdlib>
 #include <vector>
 
@@ -809,6 +810,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     (void)hipGetLastError();
     const CgWalk walk = algo == GLASMA_GAUGE_LOS_ALAMOS ? CgWalk{0, 0} : cg_walk(g, xf);
     rc = ensure_red(ctx, 16 * (size_t)nblk + 8 + 2 * kReduceTmp);
+    HostOut host(ctx, 8);
     if (!rc && algo != GLASMA_GAUGE_LOS_ALAMOS) rc = ensure_fftbuf(ctx, 8 * (size_t)g.S);  // 4 complex per site
     if (rc) return rc;
     const double* a = ctx->p.a;
@@ -819,7 +821,9 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     double* part = ctx->red;                // 2 * nblk blocks of 4 (Los Alamos: both half sweeps)
     double* spart = ctx->red + 8 * nblk;    // step monitors (Los Alamos: both half sweeps)
     double* tmp = ctx->red + 16 * nblk + 8;
-    double* h = ctx->host_out;              // host memory: the reduction writes the eight monitors straight to it
+    // the eight monitors: the reduction writes them straight to host memory
+    double* const mon = host.p ? host.p : ctx->red + 16 * nblk;
+    double h[8];
     double* F = ctx->fftbuf;
     // Los Alamos sweeps read U^G; the Fourier and Jacobi iterations form it on the fly (k_cg_dev_fused) and keep
     // the reference's lag of the top ghost layer by synchronising Gtop right after each deviation kernel, where
@@ -903,7 +907,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
         const double* const sets[2] = {part, spart};
         const long counts[2] = {!fused ? 2 * nblk : walk.zc ? (long)walk.n : nblk, fused ? nblk : 2 * nblk};
         const double mins[2] = {fm0, 0.0};
-        reduce_partials(ctx->stream, 2, sets, counts, mins, h, tmp);
+        reduce_partials(ctx->stream, 2, sets, counts, mins, mon, tmp);
         GL_HIP(ctx, hipGetLastError());
         GL_HIP(ctx, hipEventRecord(ctx->host_ev, ctx->stream));
         // On small lattices the next iteration's deviation kernel runs while the host reads this one's monitors: it
@@ -913,6 +917,8 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
         queued = fused && n + 1 < maxit && nblk <= 512;
         if (queued) deviation();
         GL_HIP(ctx, hipEventSynchronize(ctx->host_ev));
+        if (host.p) std::memcpy(h, mon, sizeof(h));
+        else GL_HIP(ctx, hipMemcpy(h, mon, sizeof(h), hipMemcpyDeviceToHost));
         gmax = h[2];
         gavg = std::sqrt(h[0] / (V * 8.0));
         fmin = h[3];
@@ -926,6 +932,7 @@ int coulomb_gauge(glasma_ctx* ctx, int algo, double tol, int maxit, double param
     if (fused) hipLaunchKernelGGL(k_cg_sync_top, grid1(g.P), dim3(kCgBlock), 0, ctx->stream, ctx->G, ctx->Gtop, g);
     if ((rc = transform_links(ctx, true))) return rc;
     GL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    host.busy = false;
     // the iteration cap reached above the tolerance: success as the reference's SetCoulombGauge returns, with a
     // message in glasma_last_error for callers that check (the reference's update cannot converge for Nz > 1)
     if (n >= maxit && gmax > tol && tol > 0.0) {

@@ -71,10 +71,7 @@ struct glasma_ctx {
     // recompute there overlaps the previous segment's backward sweep
     hipStream_t stream2 = nullptr;
     std::vector<hipEvent_t> seg_ev;
-    // pinned host memory that kernels write small results to (kHostOut doubles; pinning it takes about 60 us, so it is
-    // made with the context), and an event to wait for them
-    double* host_out = nullptr;
-    hipEvent_t host_ev = nullptr;
+    hipEvent_t host_ev = nullptr;  // a result in a HostOut is written
     std::string err;
 };
 
@@ -87,7 +84,6 @@ int hip_fail(glasma_ctx* ctx, hipError_t e, const char* what);
 // next entry point would otherwise report that stale error as their own.
 int hip_code(hipError_t e);
 int ensure_red(glasma_ctx* ctx, size_t doubles);
-constexpr long kHostOut = 8192;
 int ensure_fftbuf(glasma_ctx* ctx, size_t doubles);
 int reset_fields(glasma_ctx* ctx);
 // host array in the reference AoS layout with z ghosts (R doubles per site) <-> planes p0..p0+R-1 of a
@@ -98,6 +94,21 @@ int download_aos(glasma_ctx* ctx, const double* dev_soa, double* host_with_ghost
 void stage_context_created();
 void stage_context_destroyed();
 void stage_release_idle();
+// Pinned host memory that a call's kernels write small results to (transfer.hip), from a pool of the process: a call needs
+// it only until it has read the result.  Pinned with each context, used or not, it took 20 to 35 us of every creation
+// (8 x 8 x 16: 121-136 us with it, 102-118 without; an ensemble of 24 with one record each 28.9 and 20-24 ms).
+constexpr long kHostOut = 8192;  // doubles
+struct HostOut {
+    HostOut(const glasma_ctx* ctx, long doubles);
+    ~HostOut();
+    HostOut(const HostOut&) = delete;
+    HostOut& operator=(const HostOut&) = delete;
+    double* p = nullptr;  // null for more than kHostOut or where none can be pinned: the caller copies instead
+    bool busy = true;     // the context's stream may still write it; false once the caller has waited
+
+  private:
+    const glasma_ctx* ctx_;
+};
 void host_sync_ghosts(const glasma_ctx* ctx, double* h, int R);
 __global__ void k_set_identity(double* __restrict__ U, long S, int nmat);
 

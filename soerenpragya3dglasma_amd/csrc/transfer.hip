@@ -41,6 +41,13 @@ std::mutex g_mu;
 StageSet* g_idle[kIdleSets] = {};
 int g_contexts = 0;
 
+// the same for the memory of small results (HostOut, 64 KiB each)
+struct ResultBlock {
+    int device = -1;
+    double* p = nullptr;
+};
+ResultBlock g_results[kIdleSets];
+
 void destroy_set(StageSet* s) {
     for (int w = 0; w < kWorkers; w++) {
         if (s->stream[w]) (void)hipStreamDestroy(s->stream[w]);
@@ -176,16 +183,21 @@ void stage_context_created() {
     std::lock_guard<std::mutex> lock(g_mu);
     g_contexts++;
 }
-// gives the sets not in use back, all but `keep` of them
+// gives the sets and result blocks not in use back, all but `keep` of each
 static void release_idle(int keep) {
-    StageSet* gone[kIdleSets] = {};
+    StageSet* sets[kIdleSets] = {};
+    ResultBlock results[kIdleSets];
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        for (int i = 0; i < kIdleSets; i++)
-            if (g_idle[i] && keep-- <= 0) std::swap(gone[i], g_idle[i]);
+        for (int i = 0, n = 0; i < kIdleSets; i++)
+            if (g_idle[i] && n++ >= keep) std::swap(sets[i], g_idle[i]);
+        for (int i = 0, n = 0; i < kIdleSets; i++)
+            if (g_results[i].p && n++ >= keep) std::swap(results[i], g_results[i]);
     }
-    for (StageSet* s : gone)
+    for (StageSet* s : sets)
         if (s) destroy_set(s);
+    for (const ResultBlock& r : results)
+        if (r.p) (void)hipHostFree(r.p);
 }
 void stage_context_destroyed() {
     bool last;
@@ -196,6 +208,32 @@ void stage_context_destroyed() {
     if (last) release_idle(1);
 }
 void stage_release_idle() { release_idle(0); }
+
+HostOut::HostOut(const glasma_ctx* ctx, long doubles) : ctx_(ctx) {
+    if (doubles > kHostOut) return;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        for (ResultBlock& r : g_results)
+            if (!p && r.p && r.device == ctx->device) std::swap(p, r.p);
+    }
+    if (!p && hipHostMalloc(reinterpret_cast<void**>(&p), kHostOut * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+}
+HostOut::~HostOut() {
+    if (!p) return;
+    if (busy) (void)hipStreamSynchronize(ctx_->stream);
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        for (ResultBlock& r : g_results)
+            if (p && !r.p) {
+                std::swap(p, r.p);
+                r.device = ctx_->device;
+            }
+    }
+    if (p) (void)hipHostFree(p);
+}
 
 int upload_aos(glasma_ctx* ctx, const double* host_with_ghosts, double* dev_soa, int R, int NP, int p0) {
     return transfer<true>(ctx, const_cast<double*>(host_with_ghosts) + (size_t)ctx->g.P * R, dev_soa, R, NP < 0 ? R : NP, p0);
