@@ -42,8 +42,6 @@
 namespace glasma {
 namespace {
 
-constexpr int kCgBlock = 256;
-constexpr long kCgRound = 512;  // blocks of two waves per SIMD that the chip's 256 CUs hold at once
 
 inline dim3 grid1(long n) { return dim3((unsigned)((n + kCgBlock - 1) / kCgBlock)); }
 
@@ -364,11 +362,6 @@ __global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_fused(const double* __re
 // away.  XCD k takes the k-th eighth of the blocks, chunk by chunk: a unit's y neighbours run on the same XCD at the
 // same time.  Two waves per SIMD (at three the kernel spills and was slower than k_cg_dev_fused; reading the sites
 // x - 1, x, x + 1 together, as w_x does, spills at two and gained nothing).  Time goes into the reads' latency.
-struct CgWalk {
-    int zc;      // planes per chunk
-    unsigned n;  // blocks: units of a plane x chunks
-};
-
 template <bool CONS, bool XF>
 __global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_walk(const double* __restrict__ U, const double* __restrict__ G,
                                                            const double* __restrict__ Gtop, double* __restrict__ F,
@@ -450,30 +443,10 @@ __global__ __launch_bounds__(kCgBlock, 2) void k_cg_dev_walk(const double* __res
     block_partials(sq, fs, mx, fm, part + 4 * (long)blockIdx.x);
 }
 
-// The walk with the longest chunk, of 32, 16, 8 or 4 planes, whose blocks fill rounds of 512 (two per CU) to nine tenths,
-// else k_cg_dev_fused: a longer chunk reads fewer extra planes, but its blocks are long too, and a round that is partly
-// empty costs more than the walk saves.  With the x transforms fused in, every block must be whole (P a multiple of
-// 256).  Deviation kernel, k_cg_dev_fused against the walk with 32, 16, 8 and 4 planes (blocks): 128 x 128 x 256 696 us
-// against 638 (512), 650, 652; 64 x 64 x 256 183 against 307 (128), 177 (256), 167 (512); 125 x 125 x 250 666 against
-// 642 (496); 96 x 96 x 128 197 against 237 (144), 261 (288), 222 (576), 202 (1152); 81 x 75 x 125 127 against 141 with 4
-// (768); 100 x 100 x 100 167 against 165 with 4 (1000); 64 x 64 x 128 92 against 85 with 4 (512).
-// GLASMA_CG_WALK = planes per chunk overrides, 0 turns the walk off
+// the walk's plan (site.h cg_walk_plan); GLASMA_CG_WALK = planes per chunk overrides, 0 turns the walk off
 CgWalk cg_walk(const Geom& g, bool xf) {
     const char* e = std::getenv("GLASMA_CG_WALK");  // read per call, so that tests can set it
-    const int forced = e ? std::atoi(e) : -1;
-    if (forced == 0 || (xf && g.P % kCgBlock)) return {0, 0};
-    const long nu = (g.P + kCgBlock - 1) / kCgBlock;
-    auto blocks = [&](int c) { return nu * ((g.nz + c - 1) / c); };
-    int zc = forced > 0 ? forced : 0;
-    if (!zc)
-        for (int c : {32, 16, 8, 4})
-            if (10 * blocks(c) >= 9 * kCgRound * ((blocks(c) + kCgRound - 1) / kCgRound)) {
-                zc = c;
-                break;
-            }
-    // planes that fill their units to 7/8, and no more blocks than the partials' array has places (one per 256 sites)
-    if (!zc || 8 * g.P < 7 * nu * kCgBlock || blocks(zc) > (g.S + kCgBlock - 1) / kCgBlock) return {0, 0};
-    return {zc, (unsigned)blocks(zc)};
+    return cg_walk_plan(g, xf, e ? std::atoi(e) : -1);
 }
 
 // rows P and Q of X <- A X, A the identity outside the SU(2) block [[a, b], [c, d]] of rows / columns P, Q

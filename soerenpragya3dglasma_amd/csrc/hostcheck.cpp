@@ -54,6 +54,14 @@ void hc_row_neighbours(const int* n, long first, long* xp, long* xm) {
     }
 }
 
+// the plan of the deviation kernel that walks z: planes per chunk (0: no walk) and blocks
+void hc_cg_walk(const int* n, int xf, int forced, long* out) {
+    Geom g = {n[0], n[1], n[2], 0, (long)n[0] * n[1] * n[2], (long)n[0] * n[1]};
+    const CgWalk w = cg_walk_plan(g, xf != 0, forced);
+    out[0] = w.zc;
+    out[1] = w.n;
+}
+
 // One fused leapfrog step over tiled device-layout arrays, sequentially over sites.
 void hc_step(const int* n, const double* a, int bc, double dt, const double* U, double* Un, double* E,
              const double* J, double* Jn, double* UOld) {

@@ -4,6 +4,8 @@
 // g++) runs the very same code so that the product's arithmetic can also be exercised on a CPU.
 #pragma once
 
+#include <initializer_list>
+
 #include "su3.h"
 
 namespace glasma {
@@ -286,6 +288,38 @@ GHD long halo_site(const Geom& g, long first, int x0, int h) {
     const long end = first + kTile - 1;  // lane 63
     const long s = h == 1 ? end + 1 : end - (x0 + kTile - 1) % g.nx + g.nx - 1;
     return s < g.S ? s : g.S - 1;
+}
+
+// The gauge fixing's deviation kernel that walks z (gauge.hip k_cg_dev_walk): blocks of kCgBlock sites of a plane, zc planes
+// each.
+constexpr int kCgBlock = 256;
+constexpr long kCgRound = 512;  // blocks of two waves per SIMD that the chip's 256 CUs hold at once
+struct CgWalk {
+    int zc;      // planes per chunk; 0: no walk
+    unsigned n;  // blocks: units of a plane x chunks
+};
+// The walk with the longest chunk, of 32, 16, 8 or 4 planes, whose blocks fill rounds of 512 (two per CU) to nine tenths,
+// else k_cg_dev_fused: a longer chunk reads fewer extra planes, but its blocks are long too, and a round that is partly
+// empty costs more than the walk saves.  With the x transforms fused in, every block must be whole (P a multiple of
+// 256).  Deviation kernel, k_cg_dev_fused against the walk with 32, 16, 8 and 4 planes (blocks): 128 x 128 x 256 696 us
+// against 638 (512), 650, 652; 64 x 64 x 256 183 against 307 (128), 177 (256), 167 (512); 125 x 125 x 250 666 against
+// 642 (496); 96 x 96 x 128 197 against 237 (144), 261 (288), 222 (576), 202 (1152); 81 x 75 x 125 127 against 141 with 4
+// (768); 100 x 100 x 100 167 against 165 with 4 (1000); 64 x 64 x 128 92 against 85 with 4 (512).
+// forced: planes per chunk in place of the rule's, 0 for no walk, negative for the rule; xf: with the x transforms.
+inline CgWalk cg_walk_plan(const Geom& g, bool xf, int forced) {
+    if (forced == 0 || (xf && g.P % kCgBlock)) return {0, 0};
+    const long nu = (g.P + kCgBlock - 1) / kCgBlock;
+    auto blocks = [&](int c) { return nu * ((g.nz + c - 1) / c); };
+    int zc = forced > 0 ? forced : 0;
+    if (!zc)
+        for (int c : {32, 16, 8, 4})
+            if (10 * blocks(c) >= 9 * kCgRound * ((blocks(c) + kCgRound - 1) / kCgRound)) {
+                zc = c;
+                break;
+            }
+    // planes that fill their units to 7/8, and no more blocks than the partials' array has places (one per 256 sites)
+    if (!zc || 8 * g.P < 7 * nu * kCgBlock || blocks(zc) > (g.S + kCgBlock - 1) / kCgBlock) return {0, 0};
+    return {zc, (unsigned)blocks(zc)};
 }
 
 struct TileMap {
