@@ -52,8 +52,8 @@ __global__ void __launch_bounds__(kAdjBlock) k_vjp_local(StepAdjArgs A, long nsb
 }
 // The staple pass gives each thread one link direction (a third of the work per thread; the three directions run
 // in one launch): the own-link term and the twelve staple terms of the neighbours' E updates.
-// Measured at 48 x 48 x 128: 283 us at one wave per SIMD; the interior layers at two waves (252 registers) in one
-// launch and the two open-z boundary layers in a second took 274 + 33 us.
+// Measured at 48 x 48 x 128: 230 us at one wave per SIMD; the interior layers at two and at three waves spill (468 and
+// 1551 us).
 __global__ void __launch_bounds__(kAdjBlock) k_vjp_gather(StepAdjArgs A, long nsb) {
     long sb;
     int dir;

@@ -145,10 +145,10 @@ __device__ __forceinline__ void link_update_row(const StepArgs& A, I s, int x, i
 // The hand-over is a workgroup-scope flag: wave 3 sets it unconditionally once its stores to LDS are
 // complete, so wave 2's wait always ends; the wait is capped all the same.
 //
-// Waves 0-2 first copy U_w of the tile and of its halo sites into LDS, and the 18 of 41 link operands per site that lie on those rows are read from there.  Reading all 41 from global memory, at two
-// waves per SIMD, took 583 us at 81 x 75 x 125.
-// This takes about a third of the vector-memory accesses off the L1, whose pipeline is what the
-// kernel waits on.
+// Waves 0-2 first copy U_w of the tile and of its halo sites into LDS, and the 18 of 41 link operands per site that lie
+// on those rows are read from there.  This takes about a third of the vector-memory accesses off the L1, whose pipeline is
+// what the kernel waits on.  Reading all 41 from global memory, at two waves per SIMD, took 583 us at 81 x 75 x 125 (357
+// now).
 template <class I>
 __device__ __forceinline__ void step_tile4(const StepArgs& A, long first, StepShared<kRow>& sh) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;

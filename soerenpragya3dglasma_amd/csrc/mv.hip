@@ -10,7 +10,8 @@
 //
 // The reference walks z sequentially and solves one transverse slice at a time.  Here every transverse
 // operation (charge, smoothing, Poisson solve) runs on all z slices at once as batched 2D FFTs; only the
-// path-ordered Wilson-line product runs along z, in eight runs side by side.
+// path-ordered Wilson-line product runs along z, in eight runs side by side where the plane alone does not fill the chip
+// (scan_chunks), and not at all for the separable MV charge (k_sheet_sep).
 //
 // Work arrays (allocated for the call, freed at the end):
 //   F     complex, F[(a*Nz + z)*P + y*Nx + x], a = colour 0..7 (the FFT layout)
@@ -239,10 +240,6 @@ SheetSide sheet_side(bool right, int zlo, int zhi, int wstat, int wj) {
 __device__ __forceinline__ double mv_profile(const SheetSide& sd, int z) {
     const double u = (z - sd.center) / sd.width;
     return sd.mult_norm * (exp(-0.5 * u * u) / sqrt(2.0 * kPi * sd.width * sd.width));  // k_charge's factor
-}
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
 }
 // smoothing x Poisson over one transverse round trip: nf exp(-p^2/2 Lambda^2) p^2/(p^2+m^2) / p^2, the zero mode 0
 __device__ __forceinline__ double sheet_filter(const Geom& g, int px, int py, double ax, double ay, double lam,
@@ -1311,10 +1308,6 @@ int ic_left_vjp(glasma_ctx* ctx, const glasma_mv_params* mv, const IcTape& tape,
     return 0;
 }
 
-namespace {
-
-}  // namespace
-
 }  // namespace glasma
 
 using namespace glasma;
@@ -1323,7 +1316,7 @@ namespace glasma {
 namespace {
 // The part of reset_fields a sheet initial state needs.  The sheets write the current links, UOld and E at every
 // site (the collision's two sheets cover [0, (Nz-2)/2] and [Nz/2, Nz-1], a single nucleus all of z), and whole planes
-// of the current J (k_sheet_jstat, k_store_j); the planes of the nucleus a single-nucleus driver leaves out must be
+// of the current J (k_sheet_jstat, k_sheet_jinv); the planes of the nucleus a single-nucleus driver leaves out must be
 // zero.  The other buffers of the ping-pong pairs are written by the first step before anything reads them.
 int reset_for_sheets(glasma_ctx* ctx, int driver) {
     ctx->cur = 0;
