@@ -167,7 +167,6 @@ __device__ __forceinline__ void odd_stage(const dbl2* al, dbl2* bl, int j, int n
 // takes its inputs into registers once (a direct DFT that read LDS R^2 times took 72 us for a pass of length 100 at
 // 100 x 100 x 100, this 38; the filtered pass 239 and 95; of length 91 at 88 x 78 x 91 405 and 86), and the registers
 // that takes cost lengths without such factors (pass of length 128 at 128 x 128 x 256: 131 us against 125), hence levels.
-// The initial state's own transforms (k_sheet_plane, k_sheet_jinv), once per event, are compiled at level 2 only.
 template <bool SPLIT = false, int ODD = 0>
 __device__ __forceinline__ int stockham(dbl2* const lb, int bs, int cur, const Radices& R, int lpb, int ld,
                                         int sign, const dbl2* tw, int es = 1) {

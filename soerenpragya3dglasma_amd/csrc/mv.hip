@@ -284,7 +284,9 @@ __device__ __forceinline__ void profile_dft(double* __restrict__ prof, const She
 // What bounds this kernel is the chain of LDS stages of its one block per pair: 11 us at 16 x 16 x 32, where the separate
 // passes (load, 4 transform launches, filter, 3 profile launches, the profiles' sums by one thread per output) took 70 us
 // and their gaps, and 37 us for two nuclei of 64 x 64, where load, transforms and filter took 74 us.
+// ODD: the odd primes of nx and ny (stockham).  Compiled for all of them it took 43.6 us at 64 x 64, without 37.0.
 constexpr int kPlaneThreads = 512;
+template <int ODD>
 __global__ void __launch_bounds__(kPlaneThreads) k_sheet_plane(const double* __restrict__ xi, dbl2* __restrict__ A,
                                                                double* __restrict__ prof, Geom g, SheetSides sides,
                                                                int planes, int ld, Radices Rx, Radices Ry,
@@ -312,15 +314,15 @@ __global__ void __launch_bounds__(kPlaneThreads) k_sheet_plane(const double* __r
         lds[y * ld + i - y * g.nx] = dbl2{src[8 * i], src[8 * i + 1]};
     }
     __syncthreads();
-    int cur = stockham<false, 2>(lds, bs, 0, Rx, g.ny, ld, -1, tx);
-    cur = stockham<false, 2>(lds, bs, cur, Ry, g.nx, 1, -1, ty, ld);
+    int cur = stockham<false, ODD>(lds, bs, 0, Rx, g.ny, ld, -1, tx);
+    cur = stockham<false, ODD>(lds, bs, cur, Ry, g.nx, 1, -1, ty, ld);
     for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
         const int y = qdiv(i, g.nx, rnx), x = i - y * g.nx;
         lds[cur * bs + y * ld + x] *= sheet_filter(g, x, y, ax, ay, lam, meff);
     }
     __syncthreads();
-    cur = stockham<false, 2>(lds, bs, cur, Ry, g.nx, 1, +1, ty, ld);
-    cur = stockham<false, 2>(lds, bs, cur, Rx, g.ny, ld, +1, tx);
+    cur = stockham<false, ODD>(lds, bs, cur, Ry, g.nx, 1, +1, ty, ld);
+    cur = stockham<false, ODD>(lds, bs, cur, Rx, g.ny, ld, +1, tx);
     for (int i = threadIdx.x; i < P; i += kPlaneThreads) {
         const int y = qdiv(i, g.nx, rnx);
         A[(long)blockIdx.x * g.P + i] = lds[cur * bs + y * ld + i - y * g.nx];
@@ -576,7 +578,10 @@ __device__ __forceinline__ dbl2 jinv_factor(int pz, int nz, double az, double dt
 // LDS: two buffers of lpb * ld entries, the two-level twiddles, h(k) for k <= Nz / 2.
 // Separate passes (J-stat copied to a complex array, transform, factors, transform, real parts to J) moved 960 bytes a
 // site beyond the J-stat itself; this one moves 128.  Two nuclei at 64 x 64 x 256: 318 us before, 147 now; at
-// 256 x 256 x 512 12.6 and 6.4 ms (the LDS stages; the bytes alone would take 1.4).
+// 256 x 256 x 512 12.6 and 5.2 ms (the LDS stages; the bytes alone would take 1.4).
+// ODD: the odd primes of nz (stockham).  Compiled for all of them it took 161 us at 64 x 64 x 256 and 5.66 ms at 256 x 256
+// x 512, without 143 us and 5.19 ms.
+template <int ODD>
 __global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom g, SheetSides sides, Radices R, int lpb,
                                                     int ld, const dbl2* __restrict__ twg, double az, double dt) {
     extern __shared__ dbl2 lds[];
@@ -604,7 +609,7 @@ __global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom
             lds[li * ld + z] = v;
         }
         __syncthreads();
-        int cur = stockham<true, 2>(lds, bs, 0, R, lpb, ld, -1, tw);
+        int cur = stockham<true, ODD>(lds, bs, 0, R, lpb, ld, -1, tw);
         for (int i = threadIdx.x; i < lpb * n; i += 256) {
             const int li = i & (lpb - 1), k = i >> lg;
             dbl2 f = h[2 * k <= n ? k : n - k];
@@ -613,7 +618,7 @@ __global__ void __launch_bounds__(256) k_sheet_jinv(double* __restrict__ J, Geom
             *at = cmul(f, *at);
         }
         __syncthreads();
-        cur = stockham<true, 2>(lds, bs, cur, R, lpb, ld, +1, tw);
+        cur = stockham<true, ODD>(lds, bs, cur, R, lpb, ld, +1, tw);
         for (int i = threadIdx.x; i < lpb * n; i += 256) {
             const int li = i & (lpb - 1), z = i >> lg;
             const long s2 = s0 + li;
@@ -731,14 +736,16 @@ int sheet_currents(glasma_ctx* ctx, const double* U, const double* E, double* J,
     while (lpb > 1 && bytes(lpb) > 53 * 1024) lpb /= 2;
     const size_t lds = bytes(lpb);
     if (lds > most) return set_error(ctx, GLASMA_ERR_ARG, "the current's z line exceeds the LDS");
+    const int odd = odd_level(R);
+    const auto jinv = odd == 0 ? k_sheet_jinv<0> : odd == 1 ? k_sheet_jinv<1> : k_sheet_jinv<2>;
     if (lds > 65536)
-        GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sheet_jinv),
+        GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(jinv),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k_sheet_jstat, dim3(grid1(g.S).x, A.n), dim3(256), 0, ctx->stream, U, E, J, g, A);
     // blocks: at most 2048 a side, walking; a multiple of 8 for the XCD ranges
     const long groups = 4 * ((g.P + lpb - 1) / lpb);
     const unsigned blocks = (unsigned)(8 * std::min<long>(256, (groups + 7) / 8));
-    hipLaunchKernelGGL(k_sheet_jinv, dim3(blocks, A.n), dim3(256), lds, ctx->stream, J, g, A, R, lpb,
+    hipLaunchKernelGGL(jinv, dim3(blocks, A.n), dim3(256), lds, ctx->stream, J, g, A, R, lpb,
                        lpb > 1 ? g.nz + 1 : g.nz, tw, ctx->p.a[2], ctx->p.dt);
     GL_HIP(ctx, hipGetLastError());
     return 0;
@@ -818,15 +825,17 @@ int mv_sheets(glasma_ctx* ctx, const glasma_mv_params* mv, SheetSides A, const d
     const size_t need = sizeof(dbl2) * (2 * (size_t)g.ny * ld + g.nx + g.ny);
     const bool plane = need <= most;
     const dbl2 *twx = nullptr, *twy = nullptr;
+    const int odd = plane ? std::max(odd_level(Rx), odd_level(Ry)) : 0;
+    const auto sheet_plane = odd == 0 ? k_sheet_plane<0> : odd == 1 ? k_sheet_plane<1> : k_sheet_plane<2>;
     if (plane) {
         GL_HIP(ctx, fft_twiddles(g.nx, &twx));
         GL_HIP(ctx, fft_twiddles(g.ny, &twy));
         if (need > 65536)
-            GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sheet_plane),
+            GL_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(sheet_plane),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
     }
     const int planes = plane ? A.n : 0, wpb = kPlaneThreads / 64;
-    hipLaunchKernelGGL(k_sheet_plane, dim3(4 * planes + (A.n * g.nz + wpb - 1) / wpb), dim3(kPlaneThreads),
+    hipLaunchKernelGGL(sheet_plane, dim3(4 * planes + (A.n * g.nz + wpb - 1) / wpb), dim3(kPlaneThreads),
                        plane ? need : 0, ctx->stream, dxi, F, prof, g, A, planes, ld, Rx, Ry, twx, twy, a[0], a[1], a[2],
                        mv->lambda, mv->m_eff, dt);
     if (!plane) {

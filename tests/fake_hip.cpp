@@ -1,17 +1,20 @@
 // A stand-in for the HIP runtime, for tests of the library's host code on machines without a GPU: device memory is host
 // memory, copies are copies, kernels do nothing.  A test can refuse the n-th kernel launch and allocations beyond a
-// limit, and read how often the runtime was asked for memory, streams and launches.  Loaded with RTLD_GLOBAL before
-// libglasma.so, its functions take the place of the runtime's there.
+// limit, and read how often the runtime was asked for memory, streams and launches, and of which kernels.  Loaded with
+// RTLD_GLOBAL before libglasma.so, its functions take the place of the runtime's there.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <string>
 
 namespace {
 std::mutex mu;
 std::map<void*, size_t> device, pinned;
+std::map<const void*, std::string> kernels;  // device names of the registered kernels
+std::map<std::string, long> launched;
 long launches, refuse = -1, streams, pins, transfers_h2d, transfers_d2h;
 size_t limit = (size_t)288 << 30, shown, used, pin_limit = ~(size_t)0, pinned_bytes;
 thread_local hipError_t last = hipSuccess;
@@ -60,6 +63,13 @@ void fake_limit(size_t bytes) { limit = bytes; }
 void fake_show(size_t bytes) { shown = bytes; }  // what hipMemGetInfo calls the device's memory (0: the limit)
 void fake_pin_limit(size_t bytes) { pin_limit = bytes; }
 long fake_launches() { return launches; }
+long fake_launches_of(const char* part) {  // of kernels whose mangled name contains part
+    std::lock_guard<std::mutex> lock(mu);
+    long n = 0;
+    for (const auto& k : launched)
+        if (k.first.find(part) != std::string::npos) n += k.second;
+    return n;
+}
 long fake_streams() { return streams; }
 long fake_pins() { return pins; }
 long fake_copies() { return transfers_h2d + transfers_d2h; }
@@ -123,8 +133,9 @@ hipError_t hipGetLastError() {
     return e;
 }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "refused"; }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
     std::lock_guard<std::mutex> lock(mu);
+    launched[kernels[f]]++;
     return launches++ == refuse ? fail(hipErrorLaunchFailure) : hipSuccess;
 }
 // what a launch expression and the registration of the kernels compile to
@@ -146,7 +157,9 @@ void** __hipRegisterFatBinary(const void*) {
     static void* module = nullptr;
     return &module;
 }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+    kernels[f] = name;
+}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void**) {}
 }

@@ -9,7 +9,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PREAMBLE = """
 import ctypes, sys
 fake = ctypes.CDLL({lib!r}, mode=ctypes.RTLD_GLOBAL)
-for f in ("launches", "streams", "pins", "copies"):
+for f in ("launches", "launches_of", "streams", "pins", "copies"):
     getattr(fake, "fake_" + f).restype = ctypes.c_long
 for f in ("used", "pinned"):
     getattr(fake, "fake_" + f).restype = ctypes.c_size_t
